@@ -362,12 +362,16 @@ def _norm_on_device(gradients, order: float, maximum: float, with_mirror: bool =
     Eligible: norm_type 2 or inf; one device and one float16, bfloat16 or
     float32 gradient dtype (float64 may need the prescaled second pass);
     nothing pending on the gradients; and no cached statistics for them
-    (then the host path answers without waiting)."""
-    if order != 2.0 and not math.isinf(order):
+    (then the host path answers without waiting).  Without a mirror (nothing
+    is decided from the norm) other finite norm types too: the second pass
+    takes the prescale from the block the finalize left on the device, where
+    the host path waits for the device three times."""
+    second_pass = order != 2.0 and not math.isinf(order)
+    if second_pass and with_mirror:
         return None
     if not gradients or any(map(_PENDING, gradients)):
         return None
-    if _cached_stats(gradients) is not None:
+    if not second_pass and _cached_stats(gradients) is not None:
         return None
     groups = _device_groups(gradients)
     if len(groups) != 1:
@@ -376,12 +380,14 @@ def _norm_on_device(gradients, order: float, maximum: float, with_mirror: bool =
     if backend.adamw is None or dtype is float64:
         return None
     reject_during_capture("Host Tensor reads")           # as the host path: nothing under capture
-    plan = backend.grad_plan(gradients, dtype, incoming=True)
+    plan = backend.grad_plan(gradients, dtype, incoming=not second_pass)
     neutral = backend.neutral_ctrl()
     block = backend.empty_ctrl()                         # written whole by the finalize
     backend.grad_prepass(plan, None, neutral.data_ptr())
     mirror = runtime.take_mirror() if with_mirror else None
     backend.grad_finalize(plan, block.data_ptr(), order, maximum, 0, carry_ptr=neutral.data_ptr(), mirror=mirror)
+    if second_pass:
+        backend.grad_norm_pow(plan, block.data_ptr(), order, maximum, None)
     return backend, block, backend.ctrl_norm(block), mirror
 
 

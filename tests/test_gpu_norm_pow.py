@@ -1,0 +1,90 @@
+"""The general p-norm's second pass (``nt_grad_norm_pow``) against the oracle.
+
+``get_grad_norm`` leaves every finite norm type on the device for 16- and
+32-bit gradients; ``clip_grad_norm_`` and float64 gradients read the sums
+back.  Exponents 1, 2 and 3 sum products under a power-of-two prescale, the
+others ``pow`` under the prescale max|g|.
+
+Tolerance: the sum of n nonnegative float64 terms carries at most
+n * 2**-53 relative error in any order, a term at most 4 * 2**-53 and the
+root and the rescaling as much again: (n + 16) * 2**-53, below 1e-11 here.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import namitorch_amd as nt
+from oracle import clip as oclip
+from oracle import lowp
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+SIZES = {
+    "one": [1],
+    "edges": [3, 4, 1023, 4095, 4096, 4097, 0, 2 * 4096 + 5],
+    "many": [4096 * 9 + 1] * 3 + [17] * 40,
+}
+
+
+def _bound(grads) -> float:
+    return (sum(g.size for g in grads) + 16) * 2.0 ** -53
+
+
+def _params(grads, dtype):
+    params = [nt.Parameter(np.zeros(g.shape), dtype=dtype, device=DEV) for g in grads]
+    for p, g in zip(params, grads):
+        p.grad = nt.Tensor(g, dtype=dtype, device=DEV)
+    return params
+
+
+def _grads(sizes, dtype, sigma=1e-2):
+    rng = np.random.default_rng(41)
+    values = [rng.standard_normal(n) * sigma for n in sizes]
+    return values if dtype == "float64" else [lowp.round_to(dtype, v) for v in values]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16", "bfloat16", "float64"])
+@pytest.mark.parametrize("norm_type", [1, 3, 0.5, 2.5, 4.0])
+@pytest.mark.parametrize("sizes", sorted(SIZES))
+def test_norm_types(sizes, norm_type, dtype):
+    grads = _grads(SIZES[sizes], dtype)
+    wide = [g.astype(np.float64) for g in grads]
+    want = oclip.total_norm(wide, norm_type)
+    got = nt.optim.get_grad_norm(_params(grads, dtype), norm_type=norm_type)
+    assert got.dtype is nt.float64 and got.shape == ()
+    assert abs(got.item() - want) <= _bound(grads) * want
+    # The host path: the sums of two dtypes, combined under the larger max|g|.
+    mixed = _params(grads, dtype) + _params(_grads([5000], "float32", 3e-2), "float32")
+    want = oclip.total_norm(wide + [g.astype(np.float64) for g in _grads([5000], "float32", 3e-2)], norm_type)
+    norm = nt.optim.clip_grad_norm_(mixed, 1e300, norm_type=norm_type).item()
+    assert abs(norm - want) <= (_bound(grads) + 6000 * 2.0 ** -53) * want
+
+
+@pytest.mark.parametrize("norm_type", [1, 2, 3, 1.5, 500.0])
+@pytest.mark.parametrize("magnitude", [1e-310, 1e-200, 1.0, 1e200, 1e307])
+def test_float64_range(magnitude, norm_type):
+    """Magnitudes whose powers leave the float64 range: the prescale holds them."""
+    grads = [g * magnitude for g in _grads([1, 4097, 33], "float64", 0.3)]
+    want = oclip.total_norm(grads, norm_type)
+    got = nt.optim.get_grad_norm(_params(grads, "float64"), norm_type=norm_type).item()
+    # Subnormal results have a coarser spacing than the relative bound.
+    assert abs(got - want) <= max(2 * _bound(grads) * want, 2 * np.nextafter(0, 1)) or (np.isinf(got) and np.isinf(want))
+
+
+@pytest.mark.parametrize("bad", ["inf", "nan"])
+def test_nonfinite_and_zero(bad):
+    grads = _grads([4097, 5], "float32")
+    grads[1][2] = float(bad)
+    got = nt.optim.get_grad_norm(_params(grads, "float32"), norm_type=3).item()
+    assert np.isnan(got) if bad == "nan" else np.isinf(got)
+    assert nt.optim.get_grad_norm(_params([np.zeros(7, np.float32)], "float32"), norm_type=1).item() == 0.0
+
+
+def test_deferred_addend_is_written_back_first():
+    grads, more = _grads([4096, 9], "float32"), _grads([9, 4096], "float32")[::-1]
+    params = _params(grads, "float32")
+    nt.accumulate_grads(params, [nt.Tensor(g, device=DEV) for g in more], defer=True)
+    want = oclip.total_norm([(a + b).astype(np.float64) for a, b in zip(grads, more)], 3)
+    assert abs(nt.optim.get_grad_norm(params, norm_type=3).item() - want) <= _bound(grads) * want
