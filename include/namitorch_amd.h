@@ -318,7 +318,7 @@ int32_t nt_plan_destroy(nt_plan *plan);
  * round_to_grad_dtype(grad + incoming) as its gradient, the value the
  * accumulation would have stored, and do not write `grad`.  nt_grad_apply,
  * nt_grad_norm_pow, nt_grad_zero and nt_grad_accumulate refuse a plan with
- * any incoming pointer set (NT_ERR_VALUE).  The update is a copy queued on `stream` after the
+ * any incoming pointer set (NT_ERR_VALUE).  The update is a kernel queued on `stream` after the
  * work already queued there, so kernels launched earlier keep the old
  * pointers.  Lets one plan serve gradients that are reallocated every step
  * (Optimizer.zero_grad(set_to_none=True), optim/optimizer.py:197-206, then a

@@ -184,7 +184,6 @@ __device__ __forceinline__ void store1(typename T::raw *base, uint64_t i, float 
 }
 
 // ---- device descriptor / task tables: nt_layout.hpp ------------------------------
-constexpr int kRingSlots = 4;        // pinned slots per plan for pointer-column updates
 static_assert(kTile == kChunkQuantum, "plan chunks are whole workgroup tiles");
 
 // Per-workgroup partial of the grad pre-pass: float64 sum of squares of the

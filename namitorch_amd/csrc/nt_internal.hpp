@@ -27,14 +27,9 @@ struct nt_plan {
     nt::Partial *d_partials2;    // [max(nstage2, 1)]
     double *d_pow_partials;      // [pow_grid] (general p-norm)
     void *h_staging;             // pinned host copy of the tables (async upload source)
-    // Pointer-column updates (nt_plan_set_pointers): per-tensor alignment
-    // flags as computed at creation, and a small ring of pinned slots, each
-    // reused only after the copy that read it has completed.
+    // Per-tensor alignment flags as computed at creation, for the check of
+    // pointer-column updates (nt_plan_set_pointers).
     std::vector<uint32_t> flags;
-    void *h_ring;                // kRingSlots x ntensors pointers
-    hipEvent_t ring_events[nt::kRingSlots];
-    bool ring_used[nt::kRingSlots];
-    int32_t ring_next;
     // Descriptors whose incoming-gradient column is set: only nt_amp_prepass
     // and nt_adamw_mt (16/32-bit gradients) read that column; every other
     // entry point refuses such a plan rather than ignore the addend.
@@ -44,7 +39,7 @@ struct nt_plan {
     // the library's pools in their order when the plan is destroyed.
     hipStream_t stream;
     std::vector<hipStream_t> others;
-    uint64_t host_bytes;         // h_staging and h_ring share one page-locked buffer of this size
+    uint64_t host_bytes;         // size of h_staging
 };
 
 namespace nt {
