@@ -188,6 +188,10 @@ class DeviceStep:
             # not match then.
             clip_grad._last_stats.clear()
         self.records.clear()
+        # The gradients hold this step through their pending transform: kept
+        # here any longer, each iteration's gradients would stay in memory in
+        # a reference cycle until a garbage collection finds it.
+        self.clip_bumps.clear()
         self._reconciled = True
         self._forget()
         scheduler, self.scheduler = self.scheduler, None    # no reference cycle through it once settled

@@ -459,7 +459,7 @@ class HIPBackend:
         launch per (stored dtype, incoming dtype)."""
         by_dtypes: dict = {}
         for target, source in zip(stored, incoming):
-            by_dtypes.setdefault((target.dtype, source.dtype), []).append((target, source))
+            by_dtypes.setdefault((target._dtype, source._dtype), []).append((target, source))
         for (target_dtype, source_dtype), pairs in by_dtypes.items():
             layout = (source_dtype.code, target_dtype.code, _native.NT_DTYPE_NONE, _native.NT_DTYPE_NONE)
             rows = [(0, 0, 0, 0, 0, target._numel, 0) for target, _ in pairs]

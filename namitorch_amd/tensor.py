@@ -614,6 +614,31 @@ class Tensor:
         return f"tensor({values}, shape={self.shape}, dtype={self.dtype.name}{location}, requires_grad={self.requires_grad})"
 
 
+def device_views(flat: DeviceArray, offsets, shapes) -> list:
+    """A Tensor of each shape over `flat` from the given element offset (what
+    ``Tensor._from_storage(flat.narrow(...))`` makes, for ranges the caller
+    laid out inside `flat`)."""
+    base, start, dtype, device = flat._base, flat._ptr, flat._dtype, flat._device
+    size = dtype.itemsize
+    views = []
+    for offset, shape in zip(offsets, shapes):
+        storage = DeviceArray._make(base, start + offset * size, shape, dtype, device)
+        view = Tensor.__new__(Tensor)
+        view._storage = storage
+        view._shape = shape
+        view._dtype = dtype
+        view._device = device
+        view._ptr = storage._ptr
+        view._numel = storage._numel
+        view._requires_grad = False
+        view._grad = view._pending = view._incoming = None
+        view._clean_version = view._finite_version = view._known_item = None
+        view._version_counter = _VersionCounter()
+        view._is_leaf = True
+        views.append(view)
+    return views
+
+
 class Parameter(Tensor):
     __slots__ = ()
 
