@@ -429,6 +429,13 @@ int32_t nt_grad_norm_pow(nt_plan *plan, nt_amp_ctrl *ctrl, double norm_type,
 int32_t nt_grad_apply(nt_plan *plan, const nt_grad_xform *xform,
                       void *stream);
 
+/*
+ * nt_grad_apply for the one gradient grad[0, count) on `device`, without a
+ * plan (float32, float16 or bfloat16): the read of a single gradient.
+ */
+int32_t nt_grad_apply_flat(int32_t device, void *grad, int32_t grad_dtype, uint64_t count,
+                           const nt_grad_xform *xform, void *stream);
+
 /* Set ctrl->scale / growth_tracker and clear every other field (a kernel,
  * not a memset, so the call can be captured in a HIP graph). */
 int32_t nt_ctrl_reset(nt_amp_ctrl *ctrl, float scale, int32_t growth_tracker,

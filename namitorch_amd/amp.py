@@ -78,12 +78,13 @@ class DeviceStep:
         self.error_if_nonfinite = False
         self.error: RuntimeError | None = None
 
-    def block_for_current_stream(self):
+    def block_for_current_stream(self, current: int | None = None):
         """The control block, safe to read from work queued next on the
-        caller's current stream: a different stream first waits for this
-        step's finalize, and the block is kept from reuse until that stream's
-        work completes."""
-        current = self.backend.stream()
+        caller's current stream (`current`, when the caller has it): a
+        different stream first waits for this step's finalize, and the block
+        is kept from reuse until that stream's work completes."""
+        if current is None:
+            current = self.backend.stream()
         if self.stream is not None and current != self.stream:
             with self.backend.context():
                 _native.call("nt_stream_wait_event", current, self._ready_event().handle)

@@ -32,7 +32,7 @@ import numpy as np
 from .. import _native, runtime
 from ..array import DeviceArray
 from ..device import Device
-from ..dtype import float32, float64, int32, normalize_dtype, uint8
+from ..dtype import bfloat16, float16, float32, float64, int32, normalize_dtype, uint8
 
 PLAN_CACHE_SIZE = 16
 INCOMING = 5          # plan pointer column of deferred incoming gradients
@@ -470,6 +470,14 @@ class HIPBackend:
 
     def apply_grad_transform(self, tensors, transform) -> None:
         """Write pending GradTransforms back in place (one launch per dtype)."""
+        if len(tensors) == 1 and tensors[0]._dtype in _FLAT_APPLY:
+            # One gradient needs no plan: neither a table in device memory nor its re-pointing.
+            (tensor,) = tensors
+            stream = self.stream()
+            xform = make_xform(transform, stream=stream)
+            _native.check(_native.load().nt_grad_apply_flat(self.device.index, tensor._ptr, tensor._dtype.code,
+                                                            tensor._numel, xform, stream))
+            return
         by_dtype: dict = {}
         for tensor in tensors:
             by_dtype.setdefault(tensor.dtype, []).append(tensor)
@@ -519,8 +527,13 @@ def _is_device(value) -> bool:
     return is_device_array(value)
 
 
-def make_xform(transform, ctrl_ptr: int | None = None, honor_skip: bool = False) -> _native.GradXform:
-    """C-ABI grad transform from a GradTransform (or from a device ctrl block)."""
+_FLAT_APPLY = (float16, bfloat16, float32)
+
+
+def make_xform(transform, ctrl_ptr: int | None = None, honor_skip: bool = False,
+               stream: int | None = None) -> _native.GradXform:
+    """C-ABI grad transform from a GradTransform (or from a device ctrl block)
+    for a launch on the current stream (`stream`, when the caller has it)."""
     xform = _native.GradXform()
     xform.scale = 1.0
     xform.clip_coef = 1.0
@@ -530,7 +543,7 @@ def make_xform(transform, ctrl_ptr: int | None = None, honor_skip: bool = False)
         xform.honor_skip = int(device.honor_skip)
         # The caller launches on its current stream: another stream than the
         # one that wrote the block first waits for that step's finalize.
-        xform.ctrl = device.block_for_current_stream().data_ptr()
+        xform.ctrl = device.block_for_current_stream(stream).data_ptr()
         return xform
     if transform is not None:
         if transform.scale is not None:

@@ -781,24 +781,24 @@ template <class G> struct ApplyShape {
     static constexpr int64_t slice = G::code == NT_F32 ? (int64_t)kBlock * kVec : 0;   // 0: whole tasks
 };
 
-template <class G, int UNROLL = ApplyShape<G>::unroll, int BLOCK = kBlock>
-__global__ __launch_bounds__(BLOCK) void grad_apply_kernel(const DevTensor *__restrict__ tensors,
-                                                           const Task *__restrict__ tasks, int64_t chunk, Xform xf,
-                                                           const nt_amp_ctrl *ctrl, int32_t shift) {
+// The transform's scale and clip from a control block, when it has one;
+// false when there is nothing to apply.
+__device__ __forceinline__ bool apply_xform(const nt_amp_ctrl *ctrl, Xform &xf) {
     if (ctrl != nullptr) {
         if (xf.unscale) xf.scale = ctrl_scale_inv(ctrl->scale_used, xf.unscale, xf.inv_scale);
         xf.clip = ctrl->clip;
         xf.clip_coef = ctrl->clip_coef;
     }
-    if (!xf.unscale && !xf.clip) return;
-    const DevTensor *dp;
-    Slice slice;
-    if (!task_slice(tensors, tasks, chunk, shift, dp, slice)) return;
-    const DevTensor &d = *dp;
-    const uint64_t start = slice.start, end = slice.end;
-    auto *gp = reinterpret_cast<typename G::raw *>(d.grad);
+    return xf.unscale || xf.clip;
+}
+
+// g <- clip(unscale(g)) over gp[start, end), by one workgroup; `start` is a
+// multiple of kVec, and with `aligned` gp allows 4-element accesses.
+template <class G, int UNROLL, int BLOCK>
+__device__ __forceinline__ void apply_range(typename G::raw *gp, uint64_t start, uint64_t end, bool aligned,
+                                            const Xform &xf) {
     uint64_t scalar_from = start;
-    if (d.flags & kAligned16) {
+    if (aligned) {
         const uint64_t vend = start + ((end - start) & ~(uint64_t)(kVec - 1));
         for (uint64_t base = start + (uint64_t)threadIdx.x * kVec; base < vend; base += (uint64_t)BLOCK * kVec * UNROLL) {
             float g[UNROLL][kVec];
@@ -821,6 +821,37 @@ __global__ __launch_bounds__(BLOCK) void grad_apply_kernel(const DevTensor *__re
     }
     for (uint64_t i = scalar_from + threadIdx.x; i < end; i += BLOCK)
         store1<G>(gp, i, clip_one<G>(unscale_one<G>(load1<G>(gp, i), xf), xf));
+}
+
+template <class G, int UNROLL = ApplyShape<G>::unroll, int BLOCK = kBlock>
+__global__ __launch_bounds__(BLOCK) void grad_apply_kernel(const DevTensor *__restrict__ tensors,
+                                                           const Task *__restrict__ tasks, int64_t chunk, Xform xf,
+                                                           const nt_amp_ctrl *ctrl, int32_t shift) {
+    if (!apply_xform(ctrl, xf)) return;
+    const DevTensor *dp;
+    Slice slice;
+    if (!task_slice(tensors, tasks, chunk, shift, dp, slice)) return;
+    const DevTensor &d = *dp;
+    apply_range<G, UNROLL, BLOCK>(reinterpret_cast<typename G::raw *>(d.grad), slice.start, slice.end,
+                                  (d.flags & kAligned16) != 0u, xf);
+}
+
+// One gradient by its address, without a plan: what a program that reads its
+// gradients one by one after a clip queues per read (the launch is what costs
+// there: 148 bfloat16 gradients of GPT-2 clipped and read took 3.4 ms a pass
+// through one-tensor plans, 1.7 ms in this form).  A workgroup takes one iteration of the lanes:
+// 1024 float32 or 2048 16-bit elements, so that small gradients spread over
+// the chip.
+template <class G>
+constexpr uint64_t flat_apply_tile() { return (uint64_t)kBlock * kVec * ApplyShape<G>::unroll; }
+
+template <class G>
+__global__ __launch_bounds__(kBlock) void flat_apply_kernel(typename G::raw *gp, uint64_t count, int32_t aligned,
+                                                            Xform xf, const nt_amp_ctrl *ctrl) {
+    if (!apply_xform(ctrl, xf)) return;
+    const uint64_t start = (uint64_t)blockIdx.x * flat_apply_tile<G>();
+    const uint64_t end = min(start + flat_apply_tile<G>(), count);
+    apply_range<G, ApplyShape<G>::unroll, kBlock>(gp, start, end, aligned != 0, xf);
 }
 
 __global__ __launch_bounds__(kBlock) void grad_apply_f64_kernel(const DevTensor *__restrict__ tensors,
@@ -952,6 +983,16 @@ template <class G> struct ApplyL {
             plan->d_tensors, plan->d_tasks, plan->chunk, xf, ctrl, shift);
     }
 };
+
+template <class G>
+static int32_t launch_flat_apply(void *grad, uint64_t count, Xform xf, const nt_amp_ctrl *ctrl, hipStream_t s) {
+    const uint64_t blocks = (count + flat_apply_tile<G>() - 1) / flat_apply_tile<G>();
+    if (blocks > 0x7fffffffull) return fail(NT_ERR_VALUE, "nt_grad_apply_flat: tensor too large");
+    const int32_t aligned = (uintptr_t)grad % (kVec * sizeof(typename G::raw)) == 0 ? 1 : 0;
+    flat_apply_kernel<G><<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(static_cast<typename G::raw *>(grad), count,
+                                                                         aligned, xf, ctrl);
+    return NT_OK;
+}
 
 static uint64_t small_grid(uint64_t n) {
     uint64_t b = (n + kBlock - 1) / kBlock;
@@ -1192,6 +1233,31 @@ int32_t nt_grad_apply(nt_plan *plan, const nt_grad_xform *xform, void *stream) {
         if (rc != NT_OK) return rc;
     }
     NT_LAUNCH_CHECK("grad_apply_kernel launch");
+    return NT_OK;
+}
+
+int32_t nt_grad_apply_flat(int32_t device, void *grad, int32_t grad_dtype, uint64_t count,
+                           const nt_grad_xform *xform, void *stream) {
+    clear_error();
+    if (grad_dtype != NT_F32 && grad_dtype != NT_F16 && grad_dtype != NT_BF16)
+        return fail(NT_ERR_TYPE, "nt_grad_apply_flat: gradients must be float32, float16 or bfloat16");
+    if (xform == nullptr || count == 0) return NT_OK;
+    if (grad == nullptr) return fail(NT_ERR_VALUE, "nt_grad_apply_flat: NULL gradient");
+    if ((uintptr_t)grad % (grad_dtype == NT_F32 ? 4 : 2) != 0)
+        return fail(NT_ERR_VALUE, "nt_grad_apply_flat: gradient not aligned to its dtype");
+    DeviceGuard guard(device);
+    if (!guard.ok()) return hip_check(guard.error(), "hipSetDevice");
+    Xform xf = make_xform(xform);
+    if (xform->ctrl != nullptr) xf.unscale = xform->unscale ? 1 : 0;
+    hipStream_t s = (hipStream_t)stream;
+    int32_t rc;
+    switch (grad_dtype) {
+        case NT_F32: rc = launch_flat_apply<TF32>(grad, count, xf, xform->ctrl, s); break;
+        case NT_F16: rc = launch_flat_apply<TF16>(grad, count, xf, xform->ctrl, s); break;
+        default: rc = launch_flat_apply<TBF16>(grad, count, xf, xform->ctrl, s); break;
+    }
+    if (rc != NT_OK) return rc;
+    NT_LAUNCH_CHECK("flat_apply_kernel launch");
     return NT_OK;
 }
 
