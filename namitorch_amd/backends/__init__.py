@@ -21,10 +21,12 @@ import numpy as np
 
 from ..array import DeviceArray, is_device_array
 from ..device import Device
+from . import _graph_capture
 from ._settings import enable_fused_kernels, fused_kernels_enabled
 
 _lock = RLock()
 _backends: dict = {}
+_graph_capture.devices = _backends
 _CPU = Device("cpu")
 
 

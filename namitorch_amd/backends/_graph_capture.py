@@ -23,13 +23,17 @@ import ctypes
 from .. import _native, runtime
 
 
+# The backend registry (backends._backends: Device -> backend), which sets
+# this name; an import of it here per check would cost as much as the check.
+devices: dict = {}
+
+
 def capturing() -> bool:
     """True while the calling thread's current stream of a device with a
     HIP backend is being captured.  Before any backend exists no device
     work of this package can be in progress, so nothing is captured."""
-    from . import _backends
     status = ctypes.c_int32()
-    for device in list(_backends):
+    for device in list(devices):
         if device.type == "cpu":
             continue
         _native.call("nt_stream_capturing", runtime.current_stream(device.index), ctypes.byref(status))

@@ -68,20 +68,51 @@ def current_stream_owner(device: int):
     return stack[-1][1] if stack else None
 
 
-@contextmanager
+class _NoSwitch:
+    """Device scope of a process that sees one device: it is always current."""
+
+    __slots__ = ()
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *error):
+        return None
+
+
+class _DeviceScope:
+    __slots__ = ("index", "previous")
+
+    def __init__(self, index: int):
+        self.index = index
+
+    def __enter__(self):
+        previous = ctypes.c_int32()
+        _native.call("nt_get_device", ctypes.byref(previous))
+        self.previous = previous.value
+        if self.previous != self.index:
+            _native.call("nt_set_device", self.index)
+
+    def __exit__(self, *error):
+        if self.previous != self.index:
+            _native.call("nt_set_device", self.previous)
+
+
+_NO_SWITCH = _NoSwitch()
+_device_count = None               # devices this process sees (fixed for its life), once asked
+
+
 def device_scope(index: int):
     """Make device `index` the calling thread's current HIP device inside the
-    block (restored after), so that null-stream work lands on it."""
-    previous = ctypes.c_int32()
-    _native.call("nt_get_device", ctypes.byref(previous))
-    if previous.value == index:
-        yield
-        return
-    _native.call("nt_set_device", index)
-    try:
-        yield
-    finally:
-        _native.call("nt_set_device", previous.value)
+    block (restored after), so that null-stream work lands on it.  Every
+    launch opens one: with a single visible device, which is current on every
+    thread, nothing is asked of the runtime."""
+    global _device_count
+    if _device_count is None:
+        count = ctypes.c_int32()
+        _native.call("nt_device_count", ctypes.byref(count))
+        _device_count = count.value
+    return _NO_SWITCH if _device_count == 1 and index == 0 else _DeviceScope(index)
 
 
 class Stream:

@@ -495,13 +495,17 @@ class Tensor:
         self._ensure_inplace_allowed()
         if isinstance(src, Tensor) and src.requires_grad and is_grad_enabled():
             raise RuntimeError("copy_ from a Tensor with requires_grad=True must run inside no_grad().")
-        self[...] = src
+        self._assign(src)
         return self
 
     def __setitem__(self, index: object, value: object) -> None:
         if index is not Ellipsis:
             raise NotImplementedError("namitorch_amd Tensors support only whole-tensor assignment (t[...] = value).")
         self._ensure_inplace_allowed()
+        self._assign(value)
+
+    def _assign(self, value: object) -> None:
+        """``self[...] = value`` after ``_ensure_inplace_allowed``."""
         if isinstance(value, Tensor) and value.device != self.device:
             raise RuntimeError(f"Operands are on different devices: {self.device}, {value.device}; use an explicit .to() transfer.")
         source = value._data if isinstance(value, Tensor) else value
@@ -526,7 +530,7 @@ class Tensor:
         self._ensure_inplace_allowed()
         if isinstance(value, Tensor) and value.ndim != 0:
             raise ValueError("fill_ requires a scalar value or a zero-dimensional Tensor.")
-        self[...] = value
+        self._assign(value)
         return self
 
     # ---- conversions ---------------------------------------------------------------------
