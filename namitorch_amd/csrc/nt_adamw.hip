@@ -18,6 +18,8 @@
 // what NumPy's float16 ufuncs compute; float64 parameters use fp64.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+#include <cstring>
 #include <type_traits>
 
 #include "nt_internal.hpp"
@@ -122,6 +124,7 @@ struct MtArgs {
     int32_t honor_skip;
     int32_t split_shift;     // each task runs on 2**split_shift workgroups
     uint32_t xcd_group;      // workgroups per XCD per group of the grid order (xcd_grouped), 0: launch order
+    int32_t half_lean;       // float16 layout: every whole slice runs lean_slice_f16
 };
 
 struct MtArgs64 {
@@ -203,6 +206,104 @@ __device__ __forceinline__ void lean_slice_unscale(const DevTensor &d, const nt_
     else lean_slice<P, G, S, C, HAS_COPY, 0, CLIP>(d, c, xf, start);
 }
 
+// ---- float16 parameters: whole slices ----------------------------------------------
+// Pure float16 (parameters, gradients and moments; NumPy float16 arithmetic,
+// every operation rounded to float16) moves 14 bytes per element, half of
+// float32's, and the general loop's 100-odd VALU operations per element then
+// bound it: each fp32 operation carries two conversions, and the three
+// divides and the square root are IEEE fp32 sequences.  Here two elements go
+// per packed float16 instruction: the float16 sum or product of float16
+// values is the exact one rounded once, which is what rounding the fp32
+// result gives (24 significand bits against 11: 24 >= 2 * 11 + 2).  Divides
+// and roots take short fp32 sequences that round to the same float16:
+//  * quotient: one correction step on a * (1/b).  It is within 2^-24 (1 + 2^-20)
+//    of a/b, relatively.  A quotient of two 11-bit significands that is not a
+//    float16 rounding boundary is at least 1 / (2047 * 4095) > 2^-23 away from
+//    one, and one that is (only below the normal range) has a short
+//    significand, which the correction step gives exactly.
+//  * root: one correction step on x * rsq(x), the correctly rounded fp32 root but
+//    within 2^-45 of an fp32 tie, whose roots of 11-bit significands are
+//    2^-13 ulp away; rounding that to float16 is the double rounding the
+//    general loop has.
+// Both were checked over all float16 operands (2^32 pairs, 2^15 roots)
+// against the IEEE fp32 operation rounded to float16.
+// The pass then runs at the rate of the same loads and stores without the
+// arithmetic.  On the same buffers, general loop against this one uncapped
+// and with the cap (launch_mt):
+//   1 M elements, one tensor:         5.9, 4.4, 4.4 us
+//   30.6 M elements in 100 tensors:   85, 68.2, 66.4 us (6.5 TB/s)
+//   124.4 M elements in 148 tensors:  345, 290, 267 us (6.5 TB/s)
+constexpr int kPassSliceF16 = 512;        // 16 bytes per lane and stream on one wave
+constexpr size_t kPassLdsF16 = 10240;
+typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) u32x4v gu32x4v;
+
+// a / b rounded to float16, for float16 values (as fp32); `inv` is 1 / b to
+// within an fp32 ulp.  v_div_fixup gives the special cases.
+__device__ __forceinline__ _Float16 quotient_f16(float a, float b, float inv) {
+    float q = a * inv;
+    q = __builtin_fmaf(__builtin_fmaf(-q, b, a), inv, q);
+    return __builtin_bit_cast(_Float16, f32_to_f16(__builtin_amdgcn_div_fixupf(q, b, a)));
+}
+// sqrt(x) rounded to float16, for a float16 value.
+__device__ __forceinline__ _Float16 root_f16(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    const float r = __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+    const bool plain = x > 0.0f && x < __builtin_inff();          // not 0, inf or NaN
+    return __builtin_bit_cast(_Float16, f32_to_f16(plain ? r : (x < 0.0f ? __builtin_nanf("") : x)));
+}
+__device__ __forceinline__ half2 both(float x) { return half2{(_Float16)x, (_Float16)x}; }
+
+// One whole kPassSliceF16-element slice on one wave, of a launch with
+// MtArgs::half_lean.
+template <bool TRANSFORM>
+__device__ __forceinline__ void lean_slice_f16(const DevTensor &d, const nt_adamw_coefs &c, const Xform &xf,
+                                               uint64_t start) {
+    const uint64_t i = start + (uint64_t)threadIdx.x * 8;
+    auto *pp = reinterpret_cast<uint16_t *>(d.param) + i;
+    auto *ap = reinterpret_cast<uint16_t *>(d.exp_avg) + i;
+    auto *bp = reinterpret_cast<uint16_t *>(d.exp_avg_sq) + i;
+    const u32x4v gw = gload<true, u32x4v, gu32x4v>(reinterpret_cast<const uint16_t *>(d.grad) + i);
+    u32x4v aw = gload<true, u32x4v, gu32x4v>(ap);
+    u32x4v bw = gload<true, u32x4v, gu32x4v>(bp);
+    u32x4v pw = gload<true, u32x4v, gu32x4v>(pp);
+    const half2 beta1 = both(c.beta1), beta2 = both(c.beta2), c1 = both(c.complement1), c2 = both(c.complement2);
+    const half2 lr = both(c.lr), eps = both(c.eps), decay_factor = both(c.decay_factor);
+    const bool decay = c.weight_decay != 0.0f;
+    const float inv1 = 1.0f / c.correction1, inv2 = 1.0f / c.correction2;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        half2 g = __builtin_bit_cast(half2, (uint32_t)gw[w]);
+        if constexpr (TRANSFORM) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) g[k] = (_Float16)clip_one<TF16>(unscale_one<TF16>((float)g[k], xf), xf);
+        }
+        const half2 a = (beta1 * __builtin_bit_cast(half2, (uint32_t)aw[w])) + (c1 * g);
+        const half2 b = (beta2 * __builtin_bit_cast(half2, (uint32_t)bw[w])) + ((c2 * g) * g);
+        half2 p = __builtin_bit_cast(half2, (uint32_t)pw[w]);
+        if (decay) p = p * decay_factor;
+        half2 root, step;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            root[k] = root_f16((float)quotient_f16((float)b[k], c.correction2, inv2));
+        root = root + eps;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float corrected = (float)quotient_f16((float)a[k], c.correction1, inv1), den = (float)root[k];
+            step[k] = quotient_f16(corrected, den, __builtin_amdgcn_rcpf(den));
+        }
+        p = p - lr * step;
+        aw[w] = __builtin_bit_cast(uint32_t, a);
+        bw[w] = __builtin_bit_cast(uint32_t, b);
+        pw[w] = __builtin_bit_cast(uint32_t, p);
+    }
+    gstore<true, u32x4v, gu32x4v>(ap, aw);
+    gstore<true, u32x4v, gu32x4v>(bp, bw);
+    gstore<true, u32x4v, gu32x4v>(pp, pw);
+}
+
 // BLOCK lanes per workgroup, UNROLL 4-element groups in flight per lane;
 // each workgroup takes one slice of a task (task_slice).  A whole one-wave
 // slice in the common case runs lean_slice; everything else (tensor tails,
@@ -225,6 +326,14 @@ __global__ __launch_bounds__(BLOCK) void adamw_mt_kernel(const DevTensor *__rest
             !c.maximize && !c.coupled_weight_decay && c.update_parameter) {
             if (xf.clip) lean_slice_unscale<P, G, S, C, HAS_COPY, true>(d, c, xf, start);
             else lean_slice_unscale<P, G, S, C, HAS_COPY, false>(d, c, xf, start);
+            return;
+        }
+    }
+
+    if constexpr (BLOCK == 64 && std::is_same<R, RoundF16>::value) {
+        if (args.half_lean != 0 && end - start == (uint64_t)kPassSliceF16) {
+            if (xf.unscale == 0 && !xf.clip) lean_slice_f16<false>(d, c, xf, start);
+            else lean_slice_f16<true>(d, c, xf, start);
             return;
         }
     }
@@ -404,6 +513,32 @@ constexpr size_t pass_lds_cap() {
     else return 10240;
 }
 
+// Whether `x` is a finite float16 value.
+static bool half_value(float x) {
+    const float a = fabsf(x);
+    if (!(a <= 65504.0f)) return false;
+    uint32_t bits;
+    std::memcpy(&bits, &a, sizeof(bits));
+    if (a >= 0x1p-14f) return (bits & 0x1fffu) == 0u;            // normal: 11 significand bits
+    return a * 0x1p24f == floorf(a * 0x1p24f);                   // a multiple of the smallest
+}
+
+// Whether every slot of `plan` allows lean_slice_f16: AdamW without maximize,
+// parameters updated, and coefficients that are float16 values (the options
+// rounded to float16, but for a caller of the C ABI that passes others) with
+// bias corrections it can divide by through their inverse.
+static bool half_lean_slots(const nt_plan *plan, const MtArgs &args) {
+    for (uint32_t i = 0; i <= plan->max_slot; ++i) {
+        const nt_adamw_coefs &c = args.slots[i];
+        if (c.maximize || c.coupled_weight_decay || !c.update_parameter) return false;
+        for (float x : {c.lr, c.beta1, c.beta2, c.complement1, c.complement2, c.eps, c.weight_decay, c.decay_factor,
+                        c.correction1, c.correction2})
+            if (!half_value(x)) return false;
+        if (!(c.correction1 > 0.0f && c.correction2 > 0.0f)) return false;
+    }
+    return true;
+}
+
 // Launch shape of the pass.  A task whose size is a power-of-two multiple of
 // kPassSlice is split over one-wave workgroups of kPassSlice elements, one
 // 4-element group per lane: many short workgroups stream the pass's
@@ -415,17 +550,24 @@ constexpr size_t pass_lds_cap() {
 // order on the same buffers, 1.5 % faster on the GPT-2 list (five runs, -2.8 to
 // +0.1 %) and 3-7 % on flat 4-64 M-element tensors, while the 16-bit layouts
 // measured up to 5 % slower with any grouping, so they keep the launch order.
+//
+// Float16 launches whose slices can all run lean_slice_f16 (half_lean_slots,
+// every tensor aligned, no deferred addend) take its kPassSliceF16 slices under an occupancy
+// cap of kPassLdsF16 bytes (16 workgroups per CU); the general loop, which
+// that cap slows by a quarter, keeps kPassSlice slices and none.
 template <class P, class G, class S, class C, class R, bool HAS_COPY>
 static int32_t launch_mt(nt_plan *plan, const MtArgs &args, hipStream_t stream) {
     MtArgs a = args;
-    a.split_shift = split_shift(plan, kPassSlice);
+    constexpr bool half = std::is_same<R, RoundF16>::value;
+    if constexpr (half) a.half_lean = plan->aligned && plan->n_incoming == 0 && half_lean_slots(plan, args) ? 1 : 0;
+    a.split_shift = split_shift(plan, a.half_lean ? kPassSliceF16 : kPassSlice);
     constexpr bool all_fp32 = std::is_same<P, TF32>::value && std::is_same<G, TF32>::value &&
                               std::is_same<S, TF32>::value && !HAS_COPY;
     a.xcd_group = all_fp32 && a.split_shift > 0 ? kFp32XcdGroup : 0u;
     if (a.split_shift > 0) {
         static_assert(kPassSlice == 64 * kVec, "one 4-element group per lane of one wave");
         adamw_mt_kernel<P, G, S, C, R, HAS_COPY, 64, 1><<<dim3((unsigned)(plan->ntasks << a.split_shift)), dim3(64),
-                                                          pass_lds_cap<P, G, S>(), stream>>>(plan->d_tensors,
+                                                          a.half_lean ? kPassLdsF16 : pass_lds_cap<P, G, S>(), stream>>>(plan->d_tensors,
                                                                                              plan->d_tasks, a);
     } else {
         adamw_mt_kernel<P, G, S, C, R, HAS_COPY, kBlock, kPass2Unroll><<<dim3((unsigned)plan->ntasks), dim3(kBlock), 0,

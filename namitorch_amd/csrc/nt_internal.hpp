@@ -30,6 +30,7 @@ struct nt_plan {
     // Per-tensor alignment flags as computed at creation, for the check of
     // pointer-column updates (nt_plan_set_pointers).
     std::vector<uint32_t> flags;
+    bool aligned;                // every tensor is 16-byte aligned (kAligned16)
     // Descriptors whose incoming-gradient column is set: only nt_amp_prepass
     // and nt_adamw_mt (16/32-bit gradients) read that column; every other
     // entry point refuses such a plan rather than ignore the addend.

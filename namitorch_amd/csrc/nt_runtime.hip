@@ -227,7 +227,11 @@ int32_t nt_plan_create(int32_t device, const nt_mt_tensor *tensors, int32_t n,
     plan->pow_grid = (int32_t)(grid > 0 ? grid : 1);
 
     plan->flags.reserve((size_t)n);
-    for (int32_t t = 0; t < n; ++t) plan->flags.push_back(host[(size_t)t].flags);
+    plan->aligned = true;
+    for (int32_t t = 0; t < n; ++t) {
+        plan->flags.push_back(host[(size_t)t].flags);
+        plan->aligned = plan->aligned && (host[(size_t)t].flags & kAligned16) != 0u;
+    }
 
     hipStream_t s = (hipStream_t)stream;
     plan->stream = s;
