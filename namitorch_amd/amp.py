@@ -151,6 +151,10 @@ class DeviceStep:
                 self.mirror = None
         return self._ctrl
 
+    def read_norm(self) -> float:
+        """The block's norm, waiting for its last writer."""
+        return self.ctrl().norm
+
     def reconcile(self) -> None:
         with _settle_lock:                    # the rollback below runs once, on one thread
             self._reconcile()

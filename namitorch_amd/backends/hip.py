@@ -429,13 +429,9 @@ class HIPBackend:
             return self._neutral_ctrl
 
     def ctrl_norm(self, block: DeviceArray) -> DeviceArray:
-        """A 0-d float64 array holding the block's ``norm``, copied on the
-        device after the work queued so far (the host does not wait)."""
-        with self.context():
-            out = DeviceArray.empty((), float64, self.device)
-            _native.call("nt_memcpy_async", out.data_ptr(), block.data_ptr() + _native.AmpCtrl.norm.offset,
-                         ctypes.sizeof(ctypes.c_double), _native.NT_COPY_D2D, self.stream())
-        return out
+        """The block's ``norm`` as a 0-d float64 array: a view of the block,
+        which nothing writes after its last kernel, so no copy is queued."""
+        return DeviceArray._make(block._base, block._ptr + _native.AmpCtrl.norm.offset, (), float64, self.device)
 
     def read_ctrl(self, block: DeviceArray) -> _native.AmpCtrl:
         out = _native.AmpCtrl()

@@ -350,24 +350,24 @@ def _settle_oldest(pending: list) -> None:
     oldest.reconcile()
 
 
-def _norm_on_device(gradients, order: float, maximum: float, with_mirror: bool = False):
-    """Queue the pre-pass and a finalize over `gradients` and a device copy
-    of the norm, with no host wait: (backend, control block, 0-d float64
-    norm array, host mirror of the block or None), or None when the host
-    path must answer.  With `maximum` >= 0 the finalize also takes the clip
-    decision by the reference's rule (clip when ``max_norm / (norm + 1e-6)
-    < 1``, also for a non-finite norm).  With `with_mirror` the finalize
-    also writes the finished block to a ``runtime.take_mirror()``.
+def _norm_on_device(gradients, order: float, maximum: float):
+    """Queue the pre-pass and a finalize over `gradients`, with no host wait:
+    (backend, control block, the block's norm as a 0-d float64 array, host
+    mirror of the block or None), or None when the host path must answer.
+    With `maximum` >= 0 the finalize also takes the clip decision by the
+    reference's rule (clip when ``max_norm / (norm + 1e-6) < 1``, also for a
+    non-finite norm) and writes the finished block to a
+    ``runtime.take_mirror()``.
 
     Eligible: norm_type 2 or inf; one device and one float16, bfloat16 or
     float32 gradient dtype (float64 may need the prescaled second pass);
     nothing pending on the gradients; and no cached statistics for them
-    (then the host path answers without waiting).  Without a mirror (nothing
-    is decided from the norm) other finite norm types too: the second pass
-    takes the prescale from the block the finalize left on the device, where
-    the host path waits for the device three times."""
+    (then the host path answers without waiting).  Without a maximum other
+    finite norm types too: the second pass takes the prescale from the block
+    the finalize left on the device, where the host path waits for the device
+    three times."""
     second_pass = order != 2.0 and not math.isinf(order)
-    if second_pass and with_mirror:
+    if second_pass and maximum >= 0:
         return None
     if not gradients or any(map(_PENDING, gradients)):
         return None
@@ -384,7 +384,7 @@ def _norm_on_device(gradients, order: float, maximum: float, with_mirror: bool =
     neutral = backend.neutral_ctrl()
     block = backend.empty_ctrl()                         # written whole by the finalize
     backend.grad_prepass(plan, None, neutral.data_ptr())
-    mirror = runtime.take_mirror() if with_mirror else None
+    mirror = runtime.take_mirror() if maximum >= 0 else None
     backend.grad_finalize(plan, block.data_ptr(), order, maximum, 0, carry_ptr=neutral.data_ptr(), mirror=mirror)
     if second_pass:
         backend.grad_norm_pow(plan, block.data_ptr(), order, maximum, None)
@@ -404,7 +404,7 @@ def _clip_on_device(gradients, maximum: float, order: float) -> Tensor | None:
     can raise or differ: ``_norm_on_device``'s conditions.  (The rewrite
     itself cannot fail: every Tensor here is writable.)
     """
-    launched = _norm_on_device(gradients, order, maximum, with_mirror=True)
+    launched = _norm_on_device(gradients, order, maximum)
     if launched is None:
         return None
     backend, block, norm, mirror = launched
@@ -426,7 +426,9 @@ def _clip_on_device(gradients, maximum: float, order: float) -> Tensor | None:
     if len(_unsettled_steps) >= _UNSETTLED_LIMIT:
         _settle_oldest(_unsettled_steps)
     _unsettled_steps.append(device_step)                 # version reads settle it first
-    return Tensor._from_storage(norm, False)
+    result = Tensor._from_storage(norm, False)
+    result._known_item = (device_step.read_norm, 0)
+    return result
 
 
 def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2, error_if_nonfinite: bool = False) -> Tensor:

@@ -370,7 +370,7 @@ class Tensor:
         self._is_leaf = True
         self._clean_version = None      # version at which a state buffer was last known nonnegative
         self._finite_version = None     # version at which GradScaler last knew the gradient's finiteness
-        self._known_item = None         # (value, version): the host knows the value this device scalar was filled with
+        self._known_item = None         # (value or its reader, version): a device scalar whose value the host has or gets
 
     @classmethod
     def _from_storage(cls, storage, requires_grad: builtins.bool = False, version_counter=None,
@@ -553,12 +553,13 @@ class Tensor:
         reject_during_capture("Host Tensor reads")
         if self.size != 1:
             raise ValueError(f"item() requires exactly one element, got {self.size}.")
-        # A device scalar filled from a host value (the norm clip_grad_norm_
-        # returns) and not written since: the same value without a device
-        # round trip.  Every write through this package bumps the version.
+        # A device scalar filled from a host value, or whose kernel also
+        # writes it to the host (the norms), and not written since: the same
+        # value without a copy back.  Every write through this package bumps
+        # the version.
         known = self._known_item
         if known is not None and known[1] == self._version_counter.value:
-            return known[0]
+            return known[0]() if callable(known[0]) else known[0]
         return self.numpy().reshape(()).item()
 
     def detach(self) -> "Tensor":

@@ -88,3 +88,24 @@ def test_deferred_addend_is_written_back_first():
     nt.accumulate_grads(params, [nt.Tensor(g, device=DEV) for g in more], defer=True)
     want = oclip.total_norm([(a + b).astype(np.float64) for a, b in zip(grads, more)], 3)
     assert abs(nt.optim.get_grad_norm(params, norm_type=3).item() - want) <= _bound(grads) * want
+
+
+@pytest.mark.parametrize("norm_type", [1, 2, 3, 2.5, np.inf])
+@pytest.mark.parametrize("kind", ["finite", "zero", "inf", "nan"])
+@pytest.mark.parametrize("clip", [False, True])
+def test_item_is_the_device_scalar(norm_type, kind, clip):
+    """``.item()`` of a norm, a view of its control block or the host copy of it: the bits
+    a copy from the device gives, also again, and not after a write."""
+    grads = _grads([4097, 5], "float32")
+    if kind == "zero":
+        grads = [g * 0 for g in grads]
+    elif kind != "finite":
+        grads[0][7] = float(kind)
+    params = _params(grads, "float32")
+    norm = (nt.optim.clip_grad_norm_(params, 1e3, norm_type=norm_type) if clip
+            else nt.optim.get_grad_norm(params, norm_type=norm_type))
+    first, copied, again = norm.item(), norm.numpy(), norm.item()
+    assert type(first) is float and copied.shape == ()
+    assert np.float64(first).tobytes() == copied.tobytes() == np.float64(again).tobytes()
+    norm.fill_(7.0)
+    assert norm.item() == 7.0
