@@ -422,6 +422,17 @@ int32_t nt_grad_norm_pow(nt_plan *plan, nt_amp_ctrl *ctrl, double norm_type,
                          int32_t scale_from_ctrl, int32_t flags, void *stream);
 
 /*
+ * The p-norm (optim/clip_grad.py:70-79) of float32, float16 or bfloat16
+ * gradients for norm_type 1 or 3 in one pass over them: no prescale is
+ * needed, since the terms and their sum stay within fp64.  Adds a tensor's
+ * incoming gradient (plan column 5) first.  `ctrl` is written whole, as
+ * nt_amp_finalize writes it from `carry` (another block) without a clip or
+ * flags, with ctrl->norm the p-norm and ctrl->sumsq the sum of |g|^p.
+ */
+int32_t nt_grad_norm_sum(nt_plan *plan, nt_amp_ctrl *ctrl, const nt_amp_ctrl *carry,
+                         double norm_type, void *stream);
+
+/*
  * Write the transformed grads back in place: the deferred form of
  * GradScaler.unscale_'s grad.copy_(grad / scale) (amp.py:191) and of
  * clip_grad_norm_'s grad.copy_(f64(grad) * coef) (optim/clip_grad.py:111).

@@ -152,6 +152,7 @@ SIGNATURES = {
     "nt_amp_combine": (c_int32, [ctypes.POINTER(c_void_p), c_int32, c_void_p, c_double, c_double, c_int32, c_double,
                                  c_double, c_int32, ctypes.POINTER(c_void_p), c_void_p]),
     "nt_grad_norm_pow": (c_int32, [c_void_p, c_void_p, c_double, c_double, c_float, c_int32, c_int32, c_int32, c_void_p]),
+    "nt_grad_norm_sum": (c_int32, [c_void_p, c_void_p, c_void_p, c_double, c_void_p]),
     "nt_grad_apply": (c_int32, [c_void_p, ctypes.POINTER(GradXform), c_void_p]),
     "nt_grad_apply_flat": (c_int32, [c_int32, c_void_p, c_int32, c_uint64, ctypes.POINTER(GradXform), c_void_p]),
     "nt_grad_zero": (c_int32, [c_void_p, c_void_p]),

@@ -399,6 +399,10 @@ class HIPBackend:
                          1.0 if scale is None else scale, int(scale is not None or scale_from_ctrl),
                          int(scale_from_ctrl), int(flags), self.stream())
 
+    def grad_norm_sum(self, plan: Plan, ctrl_ptr: int, norm_type: float, carry_ptr: int) -> None:
+        with self.context():
+            _native.call("nt_grad_norm_sum", plan.handle, ctrl_ptr, carry_ptr, norm_type, self.stream())
+
     def grad_apply(self, plan: Plan, xform: _native.GradXform) -> None:
         with self.context():
             _native.call("nt_grad_apply", plan.handle, ctypes.byref(xform), self.stream())

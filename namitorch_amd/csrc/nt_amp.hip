@@ -771,6 +771,53 @@ __global__ __launch_bounds__(kBlock) void norm_pow_finalize_kernel(const double 
     *ctrl = c;
 }
 
+// ---- L1 and L3 norms of 16- and 32-bit gradients: one pass ----------------------------
+// |g|^p for p = 1 or 3 lies within [2^-447, 2^384] for every such g, and sums
+// of 2^40 terms within fp64 as well, so the norm needs no prescale and no
+// maximum beforehand: the pass keeps the statistics of the pre-pass with the
+// sum of |g|^p in the place of the squares, and the finalize takes the root.
+// 30.6 M float32 gradients in 100 tensors, p = 1, with .item(): 130 us through the
+// pre-pass and the second pass (26 and 21 us, four launches), 102 us so.
+template <class G, int P>
+__global__ __launch_bounds__(kBlock) void norm_sum_kernel(const DevTensor *__restrict__ tensors,
+                                                          const Task *__restrict__ tasks, int64_t ntasks,
+                                                          int64_t chunk, int64_t keep_from,
+                                                          Partial *__restrict__ partials) {
+    __shared__ WaveJoin join;
+    wave_join_init(join);
+    const int64_t first = (int64_t)blockIdx.x * kPrepassTasks;
+    const int64_t left = ntasks - first;
+    const int ntask = left < (int64_t)kPrepassTasks ? (int)(left > 0 ? left : 0) : kPrepassTasks;
+    PAcc acc;
+    auto one = [&](float g) {
+        const uint32_t b = f32_bits(g) & 0x7fffffffu;
+        acc.amax_bits = b > acc.amax_bits ? b : acc.amax_bits;
+        const double a = (double)bits_f32(b);
+        acc.sumsq += P == 1 ? a : a * a * a;         // infinities and NaN: the maximum tells, the sum is not used
+    };
+    prepass_visit<G>(tensors, tasks, first, ntask, chunk, keep_from,
+                     [&](const float (&g)[kPrepassUnroll][kVec]) {
+#pragma unroll
+                         for (int u = 0; u < kPrepassUnroll; ++u)
+#pragma unroll
+                             for (int k = 0; k < kVec; ++k) one(g[u][k]);
+                     },
+                     one);
+    const Partial mine{wave_sum(acc.sumsq), amax_from_bits(wave_max_u32(acc.amax_bits))};
+    wave_join_finish(join, mine, partials + blockIdx.x);
+}
+
+__global__ __launch_bounds__(kBlock) void norm_sum_finalize_kernel(const Partial *__restrict__ partials, int64_t n,
+                                                                   nt_amp_ctrl *ctrl, const nt_amp_ctrl *carry,
+                                                                   double p) {
+    Acc r = reduce_partials(partials, 0, n);
+    if (threadIdx.x != 0) return;
+    nt_amp_ctrl c = carried_ctrl(*carry);
+    decide_iteration(c, r.sumsq, r.amax, r.nan, r.inf, p, -1.0, 0, 2.0, 0.5, 1);
+    if (!c.found_inf && r.amax != 0.0) c.norm = p == 1.0 ? r.sumsq : pow(r.sumsq, 1.0 / p);
+    *ctrl = c;
+}
+
 // In-place grad transform: g <- clip(unscale(g)).  One slice (task_slice)
 // per workgroup: kBlock lanes with UNROLL 4-element groups each.  fp32
 // gradients run 1024-element slices with one group per lane; 16-bit ones,
@@ -968,6 +1015,12 @@ static int64_t keep_from_task(const nt_plan *plan) {
 template <class G> struct PrepassL {
     template <class... A> static void launch(dim3 g, hipStream_t s, A... a) {
         prepass_kernel<G><<<g, dim3(kBlock), 0, s>>>(a...);
+    }
+};
+template <class G> struct NormSumL {
+    template <class... A> static void launch(dim3 g, hipStream_t s, double p, A... a) {
+        if (p == 1.0) norm_sum_kernel<G, 1><<<g, dim3(kBlock), 0, s>>>(a...);
+        else norm_sum_kernel<G, 3><<<g, dim3(kBlock), 0, s>>>(a...);
     }
 };
 template <class G> struct NormPowL {
@@ -1209,6 +1262,38 @@ int32_t nt_grad_norm_pow(nt_plan *plan, nt_amp_ctrl *ctrl, double norm_type, dou
     norm_pow_finalize_kernel<<<dim3(1), dim3(kBlock), 0, s>>>(plan->d_pow_partials, plan->pow_grid, ctrl,
                                                               norm_type, max_norm, guard_on);
     NT_LAUNCH_CHECK("norm_pow_finalize_kernel launch");
+    return NT_OK;
+}
+
+int32_t nt_grad_norm_sum(nt_plan *plan, nt_amp_ctrl *ctrl, const nt_amp_ctrl *carry, double norm_type, void *stream) {
+    clear_error();
+    int32_t rc = check_plan(plan);
+    if (rc != NT_OK) return rc;
+    if (ctrl == nullptr || carry == nullptr) return fail(NT_ERR_VALUE, "control block is NULL");
+    if (carry == ctrl) return fail(NT_ERR_VALUE, "nt_grad_norm_sum: carry and ctrl must be different blocks");
+    if (norm_type != 1.0 && norm_type != 3.0) return fail(NT_ERR_VALUE, "nt_grad_norm_sum: norm_type must be 1 or 3");
+    if (plan->layout.grad_dtype == NT_F64)
+        return fail(NT_ERR_TYPE, "nt_grad_norm_sum: gradients must be float32, float16 or bfloat16");
+    note_stream(plan, stream);
+    DeviceGuard guard(plan->device);
+    if (!guard.ok()) return hip_check(guard.error(), "hipSetDevice");
+    hipStream_t s = (hipStream_t)stream;
+    rc = grad_dispatch<NormSumL>(plan->layout.grad_dtype, dim3((unsigned)plan->npartials), s, norm_type,
+                                 (const DevTensor *)plan->d_tensors, (const Task *)plan->d_tasks, plan->ntasks,
+                                 plan->chunk, keep_from_task(plan), plan->d_partials);
+    if (rc != NT_OK) return rc;
+    NT_LAUNCH_CHECK("norm_sum_kernel launch");
+    const Partial *src = plan->d_partials;
+    int64_t count = plan->npartials;
+    if (plan->nstage2 > 0) {
+        stage2_kernel<<<dim3((unsigned)plan->nstage2), dim3(kBlock), 0, s>>>(plan->d_partials, plan->npartials,
+                                                                            plan->d_partials2);
+        NT_LAUNCH_CHECK("stage2_kernel launch");
+        src = plan->d_partials2;
+        count = plan->nstage2;
+    }
+    norm_sum_finalize_kernel<<<dim3(1), dim3(kBlock), 0, s>>>(src, count, ctrl, carry, norm_type);
+    NT_LAUNCH_CHECK("norm_sum_finalize_kernel launch");
     return NT_OK;
 }
 

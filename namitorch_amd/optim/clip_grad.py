@@ -363,15 +363,17 @@ def _norm_on_device(gradients, order: float, maximum: float):
     float32 gradient dtype (float64 may need the prescaled second pass);
     nothing pending on the gradients; and no cached statistics for them
     (then the host path answers without waiting).  Without a maximum other
-    finite norm types too: the second pass takes the prescale from the block
-    the finalize left on the device, where the host path waits for the device
-    three times."""
-    second_pass = order != 2.0 and not math.isinf(order)
-    if second_pass and maximum >= 0:
+    finite norm types too: 1 and 3 take one pass of their own; for the others
+    the second pass takes the prescale from the block the finalize left on
+    the device, where the host path waits for the device three times."""
+    other = order != 2.0 and not math.isinf(order)
+    if other and maximum >= 0:
         return None
+    one_pass = order in (1.0, 3.0)
+    second_pass = other and not one_pass
     if not gradients or any(map(_PENDING, gradients)):
         return None
-    if not second_pass and _cached_stats(gradients) is not None:
+    if not other and _cached_stats(gradients) is not None:
         return None
     groups = _device_groups(gradients)
     if len(groups) != 1:
@@ -383,6 +385,9 @@ def _norm_on_device(gradients, order: float, maximum: float):
     plan = backend.grad_plan(gradients, dtype, incoming=not second_pass)
     neutral = backend.neutral_ctrl()
     block = backend.empty_ctrl()                         # written whole by the finalize
+    if one_pass:
+        backend.grad_norm_sum(plan, block.data_ptr(), order, neutral.data_ptr())
+        return backend, block, backend.ctrl_norm(block), None
     backend.grad_prepass(plan, None, neutral.data_ptr())
     mirror = runtime.take_mirror() if maximum >= 0 else None
     backend.grad_finalize(plan, block.data_ptr(), order, maximum, 0, carry_ptr=neutral.data_ptr(), mirror=mirror)

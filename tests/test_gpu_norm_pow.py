@@ -82,12 +82,33 @@ def test_nonfinite_and_zero(bad):
     assert nt.optim.get_grad_norm(_params([np.zeros(7, np.float32)], "float32"), norm_type=1).item() == 0.0
 
 
-def test_deferred_addend_is_written_back_first():
+@pytest.mark.parametrize("norm_type", [1, 3, 2.5])
+def test_deferred_addend_counts(norm_type):
+    """Added in the pass (1, 3) or written back before it."""
     grads, more = _grads([4096, 9], "float32"), _grads([9, 4096], "float32")[::-1]
     params = _params(grads, "float32")
     nt.accumulate_grads(params, [nt.Tensor(g, device=DEV) for g in more], defer=True)
-    want = oclip.total_norm([(a + b).astype(np.float64) for a, b in zip(grads, more)], 3)
-    assert abs(nt.optim.get_grad_norm(params, norm_type=3).item() - want) <= _bound(grads) * want
+    want = oclip.total_norm([(a + b).astype(np.float64) for a, b in zip(grads, more)], norm_type)
+    assert abs(nt.optim.get_grad_norm(params, norm_type=norm_type).item() - want) <= _bound(grads) * want
+
+
+@pytest.mark.parametrize("dtype, value", [("float32", 3.4e38), ("float32", 1e-45), ("float16", 65504.0),
+                                          ("float16", 6e-8), ("bfloat16", 3.3e38), ("bfloat16", 1e-40)])
+@pytest.mark.parametrize("norm_type", [1, 3])
+def test_extremes_of_the_narrow_types(dtype, value, norm_type):
+    """No prescale is needed: the largest and smallest values' powers stay in float64."""
+    grads = [lowp.round_to(dtype, np.full(n, value)) for n in (1, 4099)]
+    want = oclip.total_norm([g.astype(np.float64) for g in grads], norm_type)
+    got = nt.optim.get_grad_norm(_params(grads, dtype), norm_type=norm_type).item()
+    assert want > 0 and abs(got - want) <= _bound(grads) * want
+
+
+def test_many_partials_take_the_second_stage():
+    """Over 4096 workgroups of the pass."""
+    flat = nt.Tensor(np.full(4096 * 8 * 4097 + 5, 0.5, np.float16), device=DEV)
+    parameter = nt.Parameter(np.zeros(flat.shape, np.float16), device=DEV)
+    parameter.grad = flat
+    assert nt.optim.get_grad_norm([parameter], norm_type=1).item() == 0.5 * flat.size
 
 
 @pytest.mark.parametrize("norm_type", [1, 2, 3, 2.5, np.inf])
