@@ -72,6 +72,7 @@ class DeviceStep:
         self.scheduler = None                 # advanced at reconciliation iff the step updated
         self.ready = None                     # event on `stream` after the block's last writer, once needed
         self.stream = None
+        self._record = None                   # transform_record()
         # fused_step(error_if_nonfinite=True) without a scaler: a non-finite
         # norm skipped the clip and the step on the device; the reference's
         # error is kept here once the outcome is known.
@@ -90,6 +91,17 @@ class DeviceStep:
                 _native.call("nt_stream_wait_event", current, self._ready_event().handle)
                 self.block.record_stream(current)
         return self.block
+
+    def transform_record(self) -> _native.GradXform:
+        """The C-ABI record of the transform these decisions make, for
+        launches on the step's own stream; built once, since a program that
+        reads its gradients asks for it per gradient."""
+        record = self._record
+        if record is None:
+            record = _native.GradXform(scale=1.0, clip_coef=1.0, unscale=int(self.unscale),
+                                       honor_skip=int(self.honor_skip), ctrl=self.block.data_ptr())
+            self._record = record
+        return record
 
     def _ready_event(self):
         """An event on the step's stream after the block's last writer.  It is

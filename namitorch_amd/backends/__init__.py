@@ -106,6 +106,11 @@ def array_device(value) -> Device:
 
 def get_backend(value=None):
     """Backend of a Tensor, a backend array, a Device or a device string."""
+    device = getattr(value, "_device", None)
+    if type(device) is Device and hasattr(value, "_storage"):    # a Tensor (the per-launch case)
+        backend = _backends.get(device)
+        if backend is not None:
+            return backend
     if value is None or isinstance(value, (np.generic, bool, int, float)):
         target = _CPU
     elif isinstance(value, (str, Device)):

@@ -474,7 +474,9 @@ class HIPBackend:
             # One gradient needs no plan: neither a table in device memory nor its re-pointing.
             (tensor,) = tensors
             stream = self.stream()
-            xform = make_xform(transform, stream=stream)
+            device = transform.device
+            xform = device.transform_record() if device is not None and device.stream == stream \
+                else make_xform(transform, stream=stream)
             _native.check(_native.load().nt_grad_apply_flat(self.device.index, tensor._ptr, tensor._dtype.code,
                                                             tensor._numel, xform, stream))
             return

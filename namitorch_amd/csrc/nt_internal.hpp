@@ -85,6 +85,7 @@ class DeviceGuard {
 
   private:
     int prev_ = -1;
+    bool switched_ = false;
     bool ok_ = true;
     hipError_t err_ = hipSuccess;
 };

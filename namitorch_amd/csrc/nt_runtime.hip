@@ -37,15 +37,14 @@ DeviceGuard::DeviceGuard(int32_t device) {
         return;
     }
     if (prev_ != device) {
+        switched_ = true;
         err_ = hipSetDevice(device);
         ok_ = (err_ == hipSuccess);
     }
 }
 
 DeviceGuard::~DeviceGuard() {
-    int cur = -1;
-    if (prev_ >= 0 && hipGetDevice(&cur) == hipSuccess && cur != prev_ && hipSetDevice(prev_) != hipSuccess)
-        (void)hipGetLastError();
+    if (switched_ && hipSetDevice(prev_) != hipSuccess) (void)hipGetLastError();
 }
 
 Xform make_xform(const nt_grad_xform *x) {

@@ -38,6 +38,7 @@ from numbers import Real
 import numpy as np
 
 from .array import DeviceArray, is_device_array
+from .backends import get_backend
 from .backends._graph_capture import reject_during_capture
 from .device import Device
 from .dtype import (
@@ -393,12 +394,10 @@ class Tensor:
         if incoming is not None:
             check_addends([self])
             self._incoming = None
-            from .backends import get_backend
             get_backend(self).accumulate_tensors([self], [incoming[0]], assign=False)
         pending = self._pending
         if pending is None:
             return
-        from .backends import get_backend
         get_backend(self).apply_grad_transform([self], pending)
         self._pending = None
 
@@ -592,7 +591,6 @@ class Tensor:
             raise TypeError("Only floating Tensors support scalar arithmetic on the device.")
         operand = scalar_dtype(other)
         result = promote_with_scalar(self._dtype, operand)
-        from .backends import get_backend
         return get_backend(self).scalar_arithmetic(self, round_scalar(other, operand, result), op, result)
 
     def __mul__(self, other):
