@@ -1001,17 +1001,6 @@ static int32_t grad_dispatch(int32_t gdt, dim3 grid, hipStream_t s, Args... args
     return NT_OK;
 }
 
-// First pre-pass task read with temporal loads: the plan's last tasks that
-// hold at most kMallKeepBytes of gradient data (counting a deferred addend
-// stream too), so the AdamW pass re-reads them from the MALL.
-static int64_t keep_from_task(const nt_plan *plan) {
-    const int32_t gdt = plan->layout.grad_dtype;
-    const uint64_t size = gdt == NT_F16 || gdt == NT_BF16 ? 2u : 4u;
-    const uint64_t per_task = (uint64_t)plan->chunk * size * (plan->n_incoming > 0 ? 2u : 1u);
-    const int64_t keep = (int64_t)(kMallKeepBytes / per_task);
-    return plan->ntasks > keep ? plan->ntasks - keep : 0;
-}
-
 template <class G> struct PrepassL {
     template <class... A> static void launch(dim3 g, hipStream_t s, A... a) {
         prepass_kernel<G><<<g, dim3(kBlock), 0, s>>>(a...);

@@ -16,6 +16,9 @@
 
 namespace nt {
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) u32x4 gu32x4;
+
 // ---- zero ------------------------------------------------------------------------------
 // 16-byte zero stores where the tensor is aligned; a slice is one store per
 // lane of a kBlock-lane workgroup (write-only streams run fastest that way).
@@ -26,8 +29,6 @@ template <class T>
 __global__ __launch_bounds__(kBlock) void grad_zero_kernel(const DevTensor *__restrict__ tensors,
                                                            const Task *__restrict__ tasks, int64_t chunk,
                                                            int32_t shift) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(1))) u32x4 gu32x4;
     constexpr int kPer = 16 / (int)sizeof(T);           // elements per 16-byte store
     const DevTensor *dp;
     Slice slice;
@@ -54,13 +55,42 @@ __device__ __forceinline__ float accumulate_one(float stored, float incoming) {
     return D::round_f32(stored + converted);
 }
 
-// A slice is one kTile iteration: kUnroll 4-element groups per lane.  For
-// this read-read-write mix that ran faster than one-wave slices or one
-// group per lane.
+// N consecutive elements of a lane: 4, or 8 of a 16-bit type in one 16-byte access.
+template <class T, int N, bool NT> struct GroupIO : Vec4IO<T, NT> {};
+template <class T, bool NT> struct GroupIO<T, 8, NT> {
+    __device__ static void load(const uint16_t *base, uint64_t i, float (&out)[8]) {
+        const u32x4 w = gload<NT, u32x4, gu32x4>(base + i);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            out[2 * k] = T::to_f32((uint16_t)(w[k] & 0xffffu));
+            out[2 * k + 1] = T::to_f32((uint16_t)(w[k] >> 16));
+        }
+    }
+    __device__ static void store(uint16_t *base, uint64_t i, const float (&in)[8]) {
+        u32x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            w[k] = (uint32_t)T::from_f32(in[2 * k]) | ((uint32_t)T::from_f32(in[2 * k + 1]) << 16);
+        gstore<NT, u32x4, gu32x4>(base + i, w);
+    }
+};
+
+// Bound by memory.  A slice is one kTile iteration: kUnroll 4-element groups
+// per lane, or one 8-element group (16 bytes) between 16-bit types; for this
+// read-read-write mix that ran faster than one-wave slices or one 4-element
+// group per lane.  Workgroups from `keep_from` on (keep_from_task) store
+// with temporal accesses, which leave their gradients in the MALL for the
+// pre-pass; the others bypass it.  Two 8-byte groups and bypassing stores
+// everywhere against this form, 124 M float16 gradients: first accumulation
+// 81.9 -> 76.9 us (6.5 TB/s), the pre-pass after it 48.8 -> 41.0 us; adding
+// bfloat16 gradients 116.6 -> 112.6 us (6.6 TB/s).  1.3 G bfloat16 gradients:
+// 896 -> 886 us, the pre-pass level.
 template <class D, class S, bool ASSIGN>
 __global__ __launch_bounds__(kBlock) void grad_accumulate_kernel(const DevTensor *__restrict__ tensors,
                                                                  const Task *__restrict__ tasks, int64_t chunk,
-                                                                 int32_t shift) {
+                                                                 int32_t shift, uint32_t keep_from) {
+    constexpr int kGroup = sizeof(typename D::raw) == 2 && sizeof(typename S::raw) == 2 ? 8 : kVec;
+    constexpr int kGroups = kTile / (kBlock * kGroup);
     const DevTensor *dp;
     Slice slice;
     if (!task_slice(tensors, tasks, chunk, shift, dp, slice)) return;
@@ -68,27 +98,29 @@ __global__ __launch_bounds__(kBlock) void grad_accumulate_kernel(const DevTensor
     const uint64_t start = slice.start, end = slice.end;
     auto *dst = reinterpret_cast<typename D::raw *>(d.grad);
     const auto *src = reinterpret_cast<const typename S::raw *>(d.param);
+    const bool keep = blockIdx.x >= keep_from;
     uint64_t scalar_from = start;
     if (d.flags & kAligned16) {
-        const uint64_t vend = start + ((end - start) & ~(uint64_t)(kVec - 1));
-        for (uint64_t base = start + (uint64_t)threadIdx.x * kVec; base < vend; base += kTile) {
-            float a[kUnroll][kVec], b[kUnroll][kVec];
+        const uint64_t vend = start + ((end - start) & ~(uint64_t)(kGroup - 1));
+        for (uint64_t base = start + (uint64_t)threadIdx.x * kGroup; base < vend; base += kTile) {
+            float a[kGroups][kGroup], b[kGroups][kGroup];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const uint64_t i = base + (uint64_t)u * kBlock * kVec;
+            for (int u = 0; u < kGroups; ++u) {
+                const uint64_t i = base + (uint64_t)u * kBlock * kGroup;
                 if (i < vend) {
-                    Vec4IO<S, true>::load(src, i, b[u]);
-                    if constexpr (!ASSIGN) Vec4IO<D, true>::load(dst, i, a[u]);
+                    GroupIO<S, kGroup, true>::load(src, i, b[u]);
+                    if constexpr (!ASSIGN) GroupIO<D, kGroup, true>::load(dst, i, a[u]);
                 }
             }
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const uint64_t i = base + (uint64_t)u * kBlock * kVec;
+            for (int u = 0; u < kGroups; ++u) {
+                const uint64_t i = base + (uint64_t)u * kBlock * kGroup;
                 if (i < vend) {
 #pragma unroll
-                    for (int k = 0; k < kVec; ++k)
+                    for (int k = 0; k < kGroup; ++k)
                         a[u][k] = accumulate_one<D, S, ASSIGN>(ASSIGN ? 0.0f : a[u][k], b[u][k]);
-                    Vec4IO<D, true>::store(dst, i, a[u]);
+                    if (keep) GroupIO<D, kGroup, false>::store(dst, i, a[u]);
+                    else GroupIO<D, kGroup, true>::store(dst, i, a[u]);
                 }
             }
         }
@@ -154,10 +186,13 @@ template <class D, class S>
 static void launch_accumulate(const nt_plan *plan, hipStream_t s, bool assign) {
     const int32_t shift = split_shift(plan, kTile);
     const dim3 grid((unsigned)(plan->ntasks << shift));
+    const uint32_t keep_from = (uint32_t)(keep_from_task(plan) << shift);
     if (assign)
-        grad_accumulate_kernel<D, S, true><<<grid, dim3(kBlock), 0, s>>>(plan->d_tensors, plan->d_tasks, plan->chunk, shift);
+        grad_accumulate_kernel<D, S, true><<<grid, dim3(kBlock), 0, s>>>(plan->d_tensors, plan->d_tasks, plan->chunk,
+                                                                         shift, keep_from);
     else
-        grad_accumulate_kernel<D, S, false><<<grid, dim3(kBlock), 0, s>>>(plan->d_tensors, plan->d_tasks, plan->chunk, shift);
+        grad_accumulate_kernel<D, S, false><<<grid, dim3(kBlock), 0, s>>>(plan->d_tensors, plan->d_tasks, plan->chunk,
+                                                                          shift, keep_from);
 }
 
 template <class D>

@@ -68,6 +68,18 @@ inline int32_t split_shift(const nt_plan *plan, int64_t slice) {
     return shift;
 }
 
+// First task whose gradients stay in the MALL: the plan's last tasks that
+// hold at most kMallKeepBytes of gradient data (counting a deferred addend
+// stream too).  An accumulation stores them, and the pre-pass reads them,
+// with temporal accesses, so the pass after each re-reads them from there.
+inline int64_t keep_from_task(const nt_plan *plan) {
+    const int32_t gdt = plan->layout.grad_dtype;
+    const uint64_t size = gdt == NT_F16 || gdt == NT_BF16 ? 2u : 4u;
+    const uint64_t per_task = (uint64_t)plan->chunk * size * (plan->n_incoming > 0 ? 2u : 1u);
+    const int64_t keep = (int64_t)(kMallKeepBytes / per_task);
+    return plan->ntasks > keep ? plan->ntasks - keep : 0;
+}
+
 // Record `msg` as this thread's last error and return `code`.
 int32_t fail(int32_t code, const std::string &msg);
 // Convert a HIP status into NT_ERR_HIP with context; NT_OK on success.
