@@ -83,8 +83,8 @@ template <class T, bool NT> struct GroupIO<T, 8, NT> {
 // pre-pass; the others bypass it.  Two 8-byte groups and bypassing stores
 // everywhere against this form, 124 M float16 gradients: first accumulation
 // 81.9 -> 76.9 us (6.5 TB/s), the pre-pass after it 48.8 -> 41.0 us; adding
-// bfloat16 gradients 116.6 -> 112.6 us (6.6 TB/s).  1.3 G bfloat16 gradients:
-// 896 -> 886 us, the pre-pass level.
+// bfloat16 gradients 116.6 -> 112.6 us (6.6 TB/s).  1.3 G bfloat16 gradients,
+// of which the window is an eighth: 896 -> 886 us, the step level (5.50 ms).
 template <class D, class S, bool ASSIGN>
 __global__ __launch_bounds__(kBlock) void grad_accumulate_kernel(const DevTensor *__restrict__ tensors,
                                                                  const Task *__restrict__ tasks, int64_t chunk,
