@@ -55,6 +55,19 @@ constexpr int64_t kDefaultChunk = 4096;
 #define NT_LAYOUT_FN inline
 #endif
 
+// ---- grid sizes ------------------------------------------------------------------------
+// HIP takes a launch only if workgroups x lanes stays below 2**32 in each
+// dimension (hipModuleLaunchKernel), so a grid of `lanes`-lane workgroups has
+// at most this many of them: 2**24 - 1 for 256 lanes.
+NT_LAYOUT_FN constexpr uint64_t max_workgroups(uint32_t lanes) { return 0xffffffffull / lanes; }
+
+// Workgroups of a kernel that strides over `tiles` tiles by its grid: one
+// per tile, as many as a launch takes, and at least one.
+NT_LAYOUT_FN uint32_t strided_grid(uint64_t tiles, uint32_t lanes) {
+    const uint64_t most = max_workgroups(lanes);
+    return (uint32_t)(tiles < 1u ? 1u : (tiles < most ? tiles : most));
+}
+
 // ---- split launches ----------------------------------------------------------------------
 // A plan task of `chunk` elements may run on 2**shift workgroups, each taking
 // a slice of chunk >> shift elements: workgroup b covers slice

@@ -157,8 +157,10 @@ __device__ __forceinline__ typename O::raw convert(typename I::raw x) {
 // wider type (the narrower one moves 8 or 4 bytes beside them), each group
 // contiguous over the workgroup, all loads before the first store.  The grid
 // covers the array in one go: a workgroup's tile is 2 to 8 thousand elements,
-// and small arrays still spread over the chip.  Arrays that do not allow
-// these accesses, and tails, go one element per lane.
+// and small arrays still spread over the chip.  Past the largest launch
+// (strided_grid: 17 G elements with float64 on either side, 34 G with float32)
+// it strides over the array.  Arrays that do not allow these accesses, and
+// tails, go one element per lane.
 // One element per lane, through fp64, against this form (two groups and
 // nontemporal stores were the best or level of one, two and four groups with
 // either kind of store), on random data:
@@ -209,9 +211,8 @@ static void launch_cast_pair(const void *in, void *out, uint64_t n, hipStream_t 
     using S = CastShape<I, O>;
     const bool aligned = (uintptr_t)in % sizeof(typename S::in_group) == 0 &&
                          (uintptr_t)out % sizeof(typename S::out_group) == 0;
-    uint64_t blocks = (n + S::tile - 1) / S::tile;
-    if (blocks > (uint64_t(1) << 24)) blocks = uint64_t(1) << 24;
-    cast_kernel<I, O><<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(
+    const dim3 grid(strided_grid((n + S::tile - 1) / S::tile, kBlock));
+    cast_kernel<I, O><<<grid, dim3(kBlock), 0, s>>>(
         static_cast<const typename I::raw *>(in), static_cast<typename O::raw *>(out), n, aligned ? 1 : 0);
 }
 

@@ -91,7 +91,23 @@ static void test_slices_cover_each_element_once() {
     }
 }
 
+// A strided grid is one workgroup per tile while HIP takes such a launch
+// (workgroups x lanes below 2**32) and the largest it takes past that.
+static void test_strided_grids_stay_launchable() {
+    for (uint32_t lanes : {64u, 256u, 1024u}) {
+        const uint64_t most = (uint64_t(1) << 32) / lanes - 1u;
+        CHECK(max_workgroups(lanes) == most);
+        for (uint64_t tiles : {uint64_t(0), uint64_t(1), uint64_t(2), most - 1u, most, most + 1u, most + 2u,
+                               uint64_t(1) << 40, ~uint64_t(0)}) {
+            const uint64_t blocks = strided_grid(tiles, lanes);
+            CHECK(blocks >= 1u && blocks * lanes < (uint64_t(1) << 32));
+            CHECK(blocks == (tiles == 0u ? 1u : (tiles < most ? tiles : most)));
+        }
+    }
+}
+
 int main() {
+    test_strided_grids_stay_launchable();
     test_xcd_grouped_is_a_bijection();
     test_slices_cover_each_element_once();
     if (failures != 0) {
