@@ -560,7 +560,7 @@ static int32_t launch_mt(nt_plan *plan, const MtArgs &args, hipStream_t stream) 
     MtArgs a = args;
     constexpr bool half = std::is_same<R, RoundF16>::value;
     if constexpr (half) a.half_lean = plan->aligned && plan->n_incoming == 0 && half_lean_slots(plan, args) ? 1 : 0;
-    a.split_shift = split_shift(plan, a.half_lean ? kPassSliceF16 : kPassSlice);
+    a.split_shift = split_shift(plan, a.half_lean ? kPassSliceF16 : kPassSlice, 64);
     constexpr bool all_fp32 = std::is_same<P, TF32>::value && std::is_same<G, TF32>::value &&
                               std::is_same<S, TF32>::value && !HAS_COPY;
     a.xcd_group = all_fp32 && a.split_shift > 0 ? kFp32XcdGroup : 0u;
@@ -674,7 +674,7 @@ int32_t nt_adamw_mt(nt_plan *plan, const void *slots, int32_t nslots, const nt_g
         a.ctrl = xform ? xform->ctrl : nullptr;
         a.honor_skip = xform ? xform->honor_skip : 0;
         a.chunk = plan->chunk;
-        a.split_shift = split_shift(plan, kPassSlice64);
+        a.split_shift = split_shift(plan, kPassSlice64, 64);
         const dim3 grid((unsigned)(plan->ntasks << a.split_shift));
         if (a.split_shift > 0)
             adamw_mt_f64_kernel<64><<<grid, dim3(64), kPassLds64, s>>>(plan->d_tensors, plan->d_tasks, a);

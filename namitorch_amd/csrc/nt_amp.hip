@@ -1020,7 +1020,7 @@ template <class G> struct NormPowL {
 template <class G> struct ApplyL {
     // Grid: the plan's tasks, each split as ApplyShape<G> says.
     static void launch(dim3, hipStream_t s, const nt_plan *plan, Xform xf, const nt_amp_ctrl *ctrl) {
-        const int32_t shift = ApplyShape<G>::slice ? split_shift(plan, ApplyShape<G>::slice) : 0;
+        const int32_t shift = ApplyShape<G>::slice ? split_shift(plan, ApplyShape<G>::slice, kBlock) : 0;
         grad_apply_kernel<G><<<dim3((unsigned)(plan->ntasks << shift)), dim3(kBlock), 0, s>>>(
             plan->d_tensors, plan->d_tasks, plan->chunk, xf, ctrl, shift);
     }

@@ -184,7 +184,7 @@ __global__ __launch_bounds__(kBlock) void grad_accumulate_any_kernel(const DevTe
 
 template <class D, class S>
 static void launch_accumulate(const nt_plan *plan, hipStream_t s, bool assign) {
-    const int32_t shift = split_shift(plan, kTile);
+    const int32_t shift = split_shift(plan, kTile, kBlock);
     const dim3 grid((unsigned)(plan->ntasks << shift));
     const uint32_t keep_from = (uint32_t)(keep_from_task(plan) << shift);
     if (assign)
@@ -207,7 +207,7 @@ static bool dispatch_source(int32_t src, const nt_plan *plan, hipStream_t s, boo
 
 template <class T>
 static void launch_zero(const nt_plan *plan, hipStream_t s) {
-    const int32_t shift = split_shift(plan, zero_slice<T>());
+    const int32_t shift = split_shift(plan, zero_slice<T>(), kBlock);
     grad_zero_kernel<T><<<dim3((unsigned)(plan->ntasks << shift)), dim3(kBlock), 0, s>>>(plan->d_tensors, plan->d_tasks,
                                                                                        plan->chunk, shift);
 }

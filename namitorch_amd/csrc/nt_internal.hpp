@@ -56,16 +56,9 @@ __device__ __forceinline__ bool task_slice(const DevTensor *__restrict__ tensors
     return slice_of(task, b & ((1u << shift) - 1u), d->numel, chunk, shift, slice);
 }
 
-// log2(chunk / slice) when that is a power of two in [1, 64] and the grid
-// stays below 2**31 workgroups, else 0 (one workgroup per task).
-inline int32_t split_shift(const nt_plan *plan, int64_t slice) {
-    if (plan->chunk % slice != 0) return 0;
-    const int64_t parts = plan->chunk / slice;
-    if (parts > 64 || (parts & (parts - 1)) != 0) return 0;
-    int32_t shift = 0;
-    while ((int64_t(1) << shift) < parts) ++shift;
-    if (plan->ntasks > (int64_t(0x7fffffff) >> shift)) return 0;
-    return shift;
+// Split of `plan`'s tasks into `slice`-element slices on workgroups of `lanes` lanes.
+inline int32_t split_shift(const nt_plan *plan, int64_t slice, uint32_t lanes) {
+    return split_shift_of(plan->ntasks, plan->chunk, slice, lanes);
 }
 
 // First task whose gradients stay in the MALL: the plan's last tasks that

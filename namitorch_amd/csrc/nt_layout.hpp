@@ -78,6 +78,19 @@ struct Slice {
     uint64_t start, end;
 };
 
+// log2(chunk / slice) when that is a power of two in [1, 64] and HIP takes
+// a launch of that many workgroups of `lanes` lanes, else 0 (one workgroup
+// per task).
+NT_LAYOUT_FN int32_t split_shift_of(int64_t ntasks, int64_t chunk, int64_t slice, uint32_t lanes) {
+    if (chunk % slice != 0) return 0;
+    const int64_t parts = chunk / slice;
+    if (parts > 64 || (parts & (parts - 1)) != 0) return 0;
+    int32_t shift = 0;
+    while ((int64_t(1) << shift) < parts) ++shift;
+    if (ntasks > ((int64_t)max_workgroups(lanes) >> shift)) return 0;
+    return shift;
+}
+
 // The dispatcher deals the workgroups of a grid to the eight XCDs in turn
 // (workgroup b runs on XCD b mod 8).  With per_xcd > 0 the grid's work is
 // renumbered so that it is walked in groups of 8 * per_xcd workgroups and,

@@ -106,7 +106,25 @@ static void test_strided_grids_stay_launchable() {
     }
 }
 
+// A split keeps every launch below 2**32 work-items and is dropped, not
+// shortened, where it would pass them: one-wave slices of 128 float64 elements
+// at 2**21 tasks of 4096, 1024-element slices on 256 lanes at 2**22.
+static void test_splits_stay_launchable() {
+    CHECK(split_shift_of(1, 4096, 128, 64) == 5 && split_shift_of(1, 2048, 256, 64) == 3);
+    CHECK(split_shift_of(1, 4096, 4096, 256) == 0 && split_shift_of(1, 6144, 256, 64) == 0);
+    CHECK(split_shift_of(1, 65536, 512, 64) == 0 && split_shift_of(1, 32768, 512, 64) == 6);
+    CHECK(split_shift_of((int64_t(1) << 21) - 1, 4096, 128, 64) == 5 && split_shift_of(int64_t(1) << 21, 4096, 128, 64) == 0);
+    CHECK(split_shift_of((int64_t(1) << 22) - 1, 4096, 1024, 256) == 2 && split_shift_of(int64_t(1) << 22, 4096, 1024, 256) == 0);
+    for (uint32_t lanes : {64u, 256u})
+        for (int64_t slice : {128, 256, 512, 1024, 2048})
+            for (int64_t ntasks = 1; ntasks < int64_t(1) << 31; ntasks += ntasks / 3 + 1) {
+                const int32_t shift = split_shift_of(ntasks, 4096, slice, lanes);
+                CHECK(shift == 0 || ((uint64_t)ntasks << shift) * lanes < (uint64_t(1) << 32));
+            }
+}
+
 int main() {
+    test_splits_stay_launchable();
     test_strided_grids_stay_launchable();
     test_xcd_grouped_is_a_bijection();
     test_slices_cover_each_element_once();
