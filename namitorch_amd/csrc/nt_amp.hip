@@ -888,7 +888,8 @@ __global__ __launch_bounds__(BLOCK) void grad_apply_kernel(const DevTensor *__re
 // there: 148 bfloat16 gradients of GPT-2 clipped and read took 3.4 ms a pass
 // through one-tensor plans, 1.7 ms in this form).  A workgroup takes one iteration of the lanes:
 // 1024 float32 or 2048 16-bit elements, so that small gradients spread over
-// the chip.
+// the chip; past the largest launch (17 G float32 or 34 G 16-bit elements) it
+// strides over the array.
 template <class G>
 constexpr uint64_t flat_apply_tile() { return (uint64_t)kBlock * kVec * ApplyShape<G>::unroll; }
 
@@ -896,9 +897,9 @@ template <class G>
 __global__ __launch_bounds__(kBlock) void flat_apply_kernel(typename G::raw *gp, uint64_t count, int32_t aligned,
                                                             Xform xf, const nt_amp_ctrl *ctrl) {
     if (!apply_xform(ctrl, xf)) return;
-    const uint64_t start = (uint64_t)blockIdx.x * flat_apply_tile<G>();
-    const uint64_t end = min(start + flat_apply_tile<G>(), count);
-    apply_range<G, ApplyShape<G>::unroll, kBlock>(gp, start, end, aligned != 0, xf);
+    constexpr uint64_t tile = flat_apply_tile<G>();
+    for (uint64_t start = (uint64_t)blockIdx.x * tile; start < count; start += (uint64_t)gridDim.x * tile)
+        apply_range<G, ApplyShape<G>::unroll, kBlock>(gp, start, min(start + tile, count), aligned != 0, xf);
 }
 
 __global__ __launch_bounds__(kBlock) void grad_apply_f64_kernel(const DevTensor *__restrict__ tensors,
@@ -1027,13 +1028,10 @@ template <class G> struct ApplyL {
 };
 
 template <class G>
-static int32_t launch_flat_apply(void *grad, uint64_t count, Xform xf, const nt_amp_ctrl *ctrl, hipStream_t s) {
-    const uint64_t blocks = (count + flat_apply_tile<G>() - 1) / flat_apply_tile<G>();
-    if (blocks > 0x7fffffffull) return fail(NT_ERR_VALUE, "nt_grad_apply_flat: tensor too large");
+static void launch_flat_apply(void *grad, uint64_t count, Xform xf, const nt_amp_ctrl *ctrl, hipStream_t s) {
+    const dim3 grid(strided_grid((count + flat_apply_tile<G>() - 1) / flat_apply_tile<G>(), kBlock));
     const int32_t aligned = (uintptr_t)grad % (kVec * sizeof(typename G::raw)) == 0 ? 1 : 0;
-    flat_apply_kernel<G><<<dim3((unsigned)blocks), dim3(kBlock), 0, s>>>(static_cast<typename G::raw *>(grad), count,
-                                                                         aligned, xf, ctrl);
-    return NT_OK;
+    flat_apply_kernel<G><<<grid, dim3(kBlock), 0, s>>>(static_cast<typename G::raw *>(grad), count, aligned, xf, ctrl);
 }
 
 static uint64_t small_grid(uint64_t n) {
@@ -1324,13 +1322,11 @@ int32_t nt_grad_apply_flat(int32_t device, void *grad, int32_t grad_dtype, uint6
     Xform xf = make_xform(xform);
     if (xform->ctrl != nullptr) xf.unscale = xform->unscale ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;
-    int32_t rc;
     switch (grad_dtype) {
-        case NT_F32: rc = launch_flat_apply<TF32>(grad, count, xf, xform->ctrl, s); break;
-        case NT_F16: rc = launch_flat_apply<TF16>(grad, count, xf, xform->ctrl, s); break;
-        default: rc = launch_flat_apply<TBF16>(grad, count, xf, xform->ctrl, s); break;
+        case NT_F32: launch_flat_apply<TF32>(grad, count, xf, xform->ctrl, s); break;
+        case NT_F16: launch_flat_apply<TF16>(grad, count, xf, xform->ctrl, s); break;
+        default: launch_flat_apply<TBF16>(grad, count, xf, xform->ctrl, s); break;
     }
-    if (rc != NT_OK) return rc;
     NT_LAUNCH_CHECK("flat_apply_kernel launch");
     return NT_OK;
 }
