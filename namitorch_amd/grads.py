@@ -24,10 +24,11 @@ from .backends._graph_capture import reject_during_capture
 from .tensor import Tensor, device_views
 
 _GRADIENT_DTYPES = ("float16", "bfloat16", "float32", "float64")
-# First gradients of one call share allocations of about this many bytes: one
+# First gradients of one call share allocations of at most this many bytes: one
 # allocation per leaf cost 3.5 us of host time each, most of a GPT-2 iteration's
-# host time together with the checks below.  A gradient kept on its own after
-# its step keeps at most this much (or itself, if larger) from reuse.
+# host time together with the checks below.  A gradient of this size or more has
+# an allocation of its own.  So a gradient kept on its own after its step keeps
+# at most this much (or itself, if larger) from reuse.
 _ARENA_BYTES = 64 << 20
 _ARENA_ALIGN = 256          # elements: 16-byte alignment for every dtype, as the optimizer's buffers
 
@@ -169,19 +170,25 @@ def _write_back(tensors) -> None:
 
 def _fresh_gradients(parameters, backend) -> list:
     """A new gradient Tensor (contents unset) for every leaf, as views of
-    allocations of about ``_ARENA_BYTES`` per dtype."""
+    allocations of at most ``_ARENA_BYTES`` of one dtype, or of their own."""
     made: dict = {}
     runs: dict = {}
     for position, parameter in enumerate(parameters):
         dtype = parameter._dtype
+        count = -(-parameter._numel // _ARENA_ALIGN) * _ARENA_ALIGN
+        most = _ARENA_BYTES // dtype.itemsize
+        if count >= most:
+            _allocate_run(parameters, dtype, ([position], [0], parameter._numel), backend, made)
+            continue
         run = runs.get(dtype)
+        if run is not None and run[2] + count > most:
+            _allocate_run(parameters, dtype, run, backend, made)
+            run = None
         if run is None:
             run = runs[dtype] = [[], [], 0]              # positions, offsets, elements
         run[0].append(position)
         run[1].append(run[2])
-        run[2] += -(-parameter._numel // _ARENA_ALIGN) * _ARENA_ALIGN
-        if run[2] * dtype.itemsize >= _ARENA_BYTES:
-            _allocate_run(parameters, dtype, runs.pop(dtype), backend, made)
+        run[2] += count
     for dtype, run in runs.items():
         _allocate_run(parameters, dtype, run, backend, made)
     return list(map(made.__getitem__, range(len(parameters))))
