@@ -434,7 +434,9 @@ class HIPBackend:
 
     def ctrl_norm(self, block: DeviceArray) -> DeviceArray:
         """The block's ``norm`` as a 0-d float64 array: a view of the block,
-        which nothing writes after its last kernel, so no copy is queued."""
+        which nothing writes after its last kernel, so no copy is queued.
+        The caller may write it: the kernels that read the block later take
+        its clip, scale and skip fields, the host its mirror."""
         return DeviceArray._make(block._base, block._ptr + _native.AmpCtrl.norm.offset, (), float64, self.device)
 
     def read_ctrl(self, block: DeviceArray) -> _native.AmpCtrl:

@@ -383,8 +383,12 @@ class Tensor:
     # ---- storage access --------------------------------------------------------------
     @property
     def _data(self):
+        """The storage array, current.  Whoever has it may write it without
+        this Tensor's version counter noticing (another framework's view of a
+        norm, reduced over ranks), so ``item()`` reads it from here on."""
         if self._pending is not None or self._incoming is not None:
             self._materialize()
+        self._known_item = None
         return self._storage
 
     def _materialize(self) -> None:
@@ -555,7 +559,7 @@ class Tensor:
         # A device scalar filled from a host value, or whose kernel also
         # writes it to the host (the norms), and not written since: the same
         # value without a copy back.  Every write through this package bumps
-        # the version.
+        # the version; `_data`, which lets others write, forgets the value.
         known = self._known_item
         if known is not None and known[1] == self._version_counter.value:
             return known[0]() if callable(known[0]) else known[0]

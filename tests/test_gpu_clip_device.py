@@ -468,3 +468,23 @@ def test_host_known_norm_reads_without_a_device_round_trip(monkeypatch):
     assert norm.item() == 3.25 and len(reads) == 1
     scaler.step(optimizer)
     scaler.update()
+
+
+@pytest.mark.parametrize("call", [lambda p: nt.optim.clip_grad_norm_(p, 0.5), nt.optim.get_grad_norm,
+                                  lambda p: nt.optim.clip_grad_norm_(p, 0.5, error_if_nonfinite=True)])
+def test_item_sees_a_write_through_the_norms_memory(call):
+    """Another owner of the norm's memory (a reduction over ranks) writes it
+    without the Tensor: ``item()`` and ``numpy()`` agree, and the clip and the
+    step that follow are those of the norm computed."""
+    results = []
+    for write in (False, True):
+        params = [nt.Parameter(g, dtype="float32", device=DEV) for g in _grads(3, "float32")]
+        for p, g in zip(params, _grads(4, "float32", sigma=3.0)):
+            p.grad = nt.Tensor(g, dtype="float32", device=DEV)
+        norm = call(params)
+        if write:
+            norm._data.upload(np.array(123.5))
+            assert norm.item() == 123.5 and norm.numpy() == 123.5
+        nt.optim.AdamW(params).step()
+        results.append([p.numpy() for p in params] + [p.grad.numpy() for p in params])
+    assert all(_same(a, b) for a, b in zip(*results))

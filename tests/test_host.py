@@ -451,3 +451,17 @@ def test_runtime_major_version_mismatch_is_refused():
             _native._check_runtime(FakeLibrary(70226015, 60400000))
     finally:
         _native.HIP_VERSIONS = saved
+
+
+@pytest.mark.parametrize("known", [1.0, lambda: 1.0])
+def test_item_sees_writes_through_a_storage_handed_out(known):
+    """A norm's host copy serves ``item()`` only until its storage is handed
+    out: what is written there moves no version counter."""
+    norm = nt.Tensor._from_storage(np.array(1.0))
+    norm._known_item = (known, 0)
+    assert norm.item() == 1.0
+    norm._data[...] = 5.0
+    assert norm.item() == 5.0 and norm.numpy() == 5.0
+    norm._known_item = (known, 0)
+    norm.detach()._data[...] = 7.0
+    assert norm.item() == 7.0
