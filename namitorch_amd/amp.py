@@ -68,6 +68,7 @@ class DeviceStep:
         self.mirror = mirror
         self.launched = False                 # a kernel that writes `mirror` was queued
         self._ctrl = None
+        self._waiting = 0                     # threads in _await_block()
         self._reconciled = False
         self.scheduler = None                 # advanced at reconciliation iff the step updated
         self.ready = None                     # event on `stream` after the block's last writer, once needed
@@ -145,8 +146,38 @@ class DeviceStep:
                 return
 
     def ctrl(self) -> _native.AmpCtrl:
+        mirror = self.mirror
+        if self._ctrl is None and (mirror is None or not mirror.ready):
+            self._await_block()
         with _settle_lock:                    # one reader takes the mirror and gives it back
             return self._read_ctrl()
+
+    def _await_block(self) -> None:
+        """Wait for the block's last writer without holding the lock, so that
+        a thread that reads this step's outcome keeps no other from settling
+        its own.  The mirror is not given back while a thread waits on it."""
+        with _settle_lock:
+            if self._ctrl is not None:
+                return
+            mirror = self.mirror
+            event = self._ready_event() if mirror is None else None
+            self._waiting += 1
+        try:
+            if event is not None:
+                event.synchronize()
+            else:
+                with self.backend.context():
+                    _native.call("nt_mirror_wait", ctypes.addressof(mirror), self.stream)
+        finally:
+            with _settle_lock:
+                self._waiting -= 1
+                self._give_mirror()
+
+    def _give_mirror(self) -> None:
+        """Return the mirror to the pool once it is read and no thread waits on it."""
+        if self.mirror is not None and self._ctrl is not None and not self._waiting:
+            runtime.give_mirror(self.mirror)
+            self.mirror = None
 
     def _read_ctrl(self) -> _native.AmpCtrl:
         if self._ctrl is None:
@@ -159,8 +190,7 @@ class DeviceStep:
                     with self.backend.context():
                         _native.call("nt_mirror_wait", ctypes.addressof(mirror), self.stream)
                 self._ctrl = _native.AmpCtrl.from_buffer_copy(mirror)
-                runtime.give_mirror(mirror)
-                self.mirror = None
+                self._give_mirror()
         return self._ctrl
 
     def read_norm(self) -> float:
