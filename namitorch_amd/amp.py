@@ -205,7 +205,7 @@ class DeviceStep:
         if self._reconciled:
             self._forget()                    # settled: never left waiting in the unsettled list
             return
-        ctrl = self.ctrl()
+        ctrl = self._read_ctrl()              # the lock is held already
         if self.honor_skip and ctrl.skip:
             # The AdamW pass left everything untouched: undo the host bookkeeping.
             for parameter, state, first, second, master, step, bumped, moved in self.records:
