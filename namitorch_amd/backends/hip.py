@@ -333,9 +333,15 @@ class HIPBackend:
             if plan.columns.get(column) == values:
                 continue
             array = (ctypes.c_void_p * max(1, len(values)))(*values)
+            # A failed update may have rewritten part of the column: until one
+            # succeeds, the plan holds no known pointers.  A refused one
+            # (NT_ERR_VALUE) changed nothing.
+            held = plan.columns.pop(column, None)
             with self.context():
                 status = _native.load().nt_plan_set_pointers(plan.handle, column, array, len(values), stream)
             if status == _native.NT_ERR_VALUE:
+                if held is not None:
+                    plan.columns[column] = held
                 return False
             _native.check(status)
             plan.columns[column] = values

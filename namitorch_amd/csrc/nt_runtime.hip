@@ -324,6 +324,10 @@ int32_t nt_plan_set_pointers(nt_plan *plan, int32_t column, const void *const *p
     DeviceGuard guard(plan->device);
     if (!guard.ok()) return hip_check(guard.error(), "hipSetDevice");
     hipStream_t s = (hipStream_t)stream;
+    // A list of several launches can fail between them: until the last is
+    // queued the plan counts as one with addends, which every entry point
+    // that would ignore them refuses.
+    if (column == kIncomingColumn) plan->n_incoming = n;
     for (int32_t first = 0; first < n; first += kWidePointers) {
         const int32_t count = n - first < kWidePointers ? n - first : kWidePointers;
         rc = count <= kFewPointers ? launch_pointers<kFewPointers>(plan, column, pointers, first, count, s)
