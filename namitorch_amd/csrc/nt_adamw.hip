@@ -18,10 +18,9 @@
 // what NumPy's float16 ufuncs compute; float64 parameters use fp64.
 #include <hip/hip_runtime.h>
 
-#include <cmath>
-#include <cstring>
 #include <type_traits>
 
+#include "nt_half.hpp"
 #include "nt_internal.hpp"
 
 namespace nt {
@@ -225,8 +224,9 @@ __device__ __forceinline__ void lean_slice_unscale(const DevTensor &d, const nt_
 //    within 2^-45 of an fp32 tie, whose roots of 11-bit significands are
 //    2^-13 ulp away; rounding that to float16 is the double rounding the
 //    general loop has.
-// Both were checked over all float16 operands (2^32 pairs, 2^15 roots)
-// against the IEEE fp32 operation rounded to float16.
+// The steps are quotient_step and root_step of nt_half.hpp; its host test runs
+// all significand pairs and all roots through them against the IEEE fp32
+// operation, with reciprocals off by -1, 0 and +1 fp32 ulp.
 // The pass then runs at the rate of the same loads and stores without the
 // arithmetic.  On the same buffers, general loop against this one uncapped
 // and with the cap (launch_mt):
@@ -242,15 +242,11 @@ typedef __attribute__((address_space(1))) u32x4v gu32x4v;
 // a / b rounded to float16, for float16 values (as fp32); `inv` is 1 / b to
 // within an fp32 ulp.  v_div_fixup gives the special cases.
 __device__ __forceinline__ _Float16 quotient_f16(float a, float b, float inv) {
-    float q = a * inv;
-    q = __builtin_fmaf(__builtin_fmaf(-q, b, a), inv, q);
-    return __builtin_bit_cast(_Float16, f32_to_f16(__builtin_amdgcn_div_fixupf(q, b, a)));
+    return __builtin_bit_cast(_Float16, f32_to_f16(__builtin_amdgcn_div_fixupf(quotient_step(a, b, inv), b, a)));
 }
 // sqrt(x) rounded to float16, for a float16 value.
 __device__ __forceinline__ _Float16 root_f16(float x) {
-    const float y = __builtin_amdgcn_rsqf(x);
-    const float s = x * y;
-    const float r = __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+    const float r = root_step(x, __builtin_amdgcn_rsqf(x));
     const bool plain = x > 0.0f && x < __builtin_inff();          // not 0, inf or NaN
     return __builtin_bit_cast(_Float16, f32_to_f16(plain ? r : (x < 0.0f ? __builtin_nanf("") : x)));
 }
@@ -513,32 +509,6 @@ constexpr size_t pass_lds_cap() {
     else return 10240;
 }
 
-// Whether `x` is a finite float16 value.
-static bool half_value(float x) {
-    const float a = fabsf(x);
-    if (!(a <= 65504.0f)) return false;
-    uint32_t bits;
-    std::memcpy(&bits, &a, sizeof(bits));
-    if (a >= 0x1p-14f) return (bits & 0x1fffu) == 0u;            // normal: 11 significand bits
-    return a * 0x1p24f == floorf(a * 0x1p24f);                   // a multiple of the smallest
-}
-
-// Whether every slot of `plan` allows lean_slice_f16: AdamW without maximize,
-// parameters updated, and coefficients that are float16 values (the options
-// rounded to float16, but for a caller of the C ABI that passes others) with
-// bias corrections it can divide by through their inverse.
-static bool half_lean_slots(const nt_plan *plan, const MtArgs &args) {
-    for (uint32_t i = 0; i <= plan->max_slot; ++i) {
-        const nt_adamw_coefs &c = args.slots[i];
-        if (c.maximize || c.coupled_weight_decay || !c.update_parameter) return false;
-        for (float x : {c.lr, c.beta1, c.beta2, c.complement1, c.complement2, c.eps, c.weight_decay, c.decay_factor,
-                        c.correction1, c.correction2})
-            if (!half_value(x)) return false;
-        if (!(c.correction1 > 0.0f && c.correction2 > 0.0f)) return false;
-    }
-    return true;
-}
-
 // Launch shape of the pass.  A task whose size is a power-of-two multiple of
 // kPassSlice is split over one-wave workgroups of kPassSlice elements, one
 // 4-element group per lane: many short workgroups stream the pass's
@@ -559,7 +529,7 @@ template <class P, class G, class S, class C, class R, bool HAS_COPY>
 static int32_t launch_mt(nt_plan *plan, const MtArgs &args, hipStream_t stream) {
     MtArgs a = args;
     constexpr bool half = std::is_same<R, RoundF16>::value;
-    if constexpr (half) a.half_lean = plan->aligned && plan->n_incoming == 0 && half_lean_slots(plan, args) ? 1 : 0;
+    if constexpr (half) a.half_lean = plan->aligned && plan->n_incoming == 0 && half_lean_slots(args.slots, plan->max_slot + 1u) ? 1 : 0;
     a.split_shift = split_shift(plan, a.half_lean ? kPassSliceF16 : kPassSlice, 64);
     constexpr bool all_fp32 = std::is_same<P, TF32>::value && std::is_same<G, TF32>::value &&
                               std::is_same<S, TF32>::value && !HAS_COPY;

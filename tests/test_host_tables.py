@@ -1,6 +1,7 @@
 """Host unit tests of the library's plain C++ parts — the plan-table builder,
 the caching memory pools, the GradScaler / clip decisions the finalize
-kernels make and the kernels' workgroup -> element arithmetic — compiled
+kernels make, the kernels' workgroup -> element arithmetic and the float16
+pass's — compiled
 with g++ under AddressSanitizer and UndefinedBehaviorSanitizer (no GPU
 involved)."""
 
@@ -52,3 +53,10 @@ def test_workgroup_layout_under_sanitizers(tmp_path):
     """Header-only: nt_layout.hpp's XCD-grouped grid renumbering (a bijection
     for every grid size) and task slicing (each element exactly once)."""
     _run_sanitized(tmp_path, "layout_test.cpp", None)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is not installed")
+def test_float16_arithmetic_under_sanitizers(tmp_path):
+    """Header-only: nt_half.hpp's quotient and root steps over every pair of
+    float16 significands and every root, and the rule that selects them."""
+    _run_sanitized(tmp_path, "half_test.cpp", None)
