@@ -156,11 +156,11 @@ __device__ __forceinline__ typename O::raw convert(typename I::raw x) {
 // every access is wide: a lane takes kCastUnroll groups of 16 bytes of the
 // wider type (the narrower one moves 8 or 4 bytes beside them), each group
 // contiguous over the workgroup, all loads before the first store.  The grid
-// covers the array in one go: a workgroup's tile is 2 to 8 thousand elements,
-// and small arrays still spread over the chip.  Past the largest launch
-// (strided_grid: 17 G elements with float64 on either side, 34 G with float32)
-// it strides over the array.  Arrays that do not allow these accesses, and
-// tails, go one element per lane.
+// covers the array in one go: a workgroup's tile is 1024 elements with float64
+// on either side, 2048 with float32 and 4096 between 16-bit types, so small
+// arrays still spread over the chip.  Past the largest launch (strided_grid:
+// 17, 34 and 69 G elements) it strides over the array.  Arrays that do not
+// allow these accesses, and tails, go one element per lane.
 // One element per lane, through fp64, against this form (two groups and
 // nontemporal stores were the best or level of one, two and four groups with
 // either kind of store), on random data:

@@ -1,6 +1,7 @@
-"""``nt_cast`` at the edges of its tiles (512 to 4096 elements by type pair),
-for tails and for arrays that do not allow 16-byte accesses: NumPy's cast
-with one rounding, special values included."""
+"""``nt_cast`` at the edges of its tiles (1024 elements with float64 on either
+side, 2048 with float32, 4096 between 16-bit types), for tails and for arrays
+that do not allow 16-byte accesses: NumPy's cast with one rounding, special
+values included."""
 
 from __future__ import annotations
 
@@ -22,7 +23,7 @@ SPECIAL = [0.0, -0.0, 1.0, -1.0, 65504.0, 65520.0, 3.4e38, 1e-8, -1e-45, 6e-8, n
 def test_values_and_tile_edges(source, target):
     if source == target:
         pytest.skip("a copy")
-    for count in (1, 20, 511, 512, 513, 1024, 2047, 2048, 2049, 4096, 4097, 12289):
+    for count in (1, 20, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 12289):
         rng = np.random.default_rng(count)
         host = rng.standard_normal(count + 3) * np.exp2(rng.integers(-30, 17, count + 3))
         host[:min(count, 20)] = SPECIAL[:min(count, 20)]

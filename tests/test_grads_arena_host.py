@@ -14,6 +14,7 @@ from namitorch_amd.array import DeviceArray
 from namitorch_amd.device import Device
 from namitorch_amd.dtype import normalize_dtype
 from namitorch_amd.runtime import _NoSwitch
+from namitorch_amd.tensor import Tensor
 
 DEVICE = Device("cuda", 0)
 BACKEND = SimpleNamespace(device=DEVICE, context=_NoSwitch)
@@ -72,3 +73,13 @@ def test_bound_on_any_list(fresh, monkeypatch, seed):
     # Two neighbours of one dtype that fit together share: at most about twice the fewest allocations.
     total = sum(-(-leaf._numel // 256) * 256 * leaf._dtype.itemsize for leaf in leaves)
     assert len(blocks) <= 2 * (total // (1 << 16)) + 8
+
+
+def test_views_are_whole_tensors(fresh):
+    """``device_views`` fills every slot as the constructor does."""
+    (view, _), _ = fresh([_leaf(300, "float16"), _leaf(5, "float16")])
+    made = Tensor._from_storage(view._storage)
+    for slot in Tensor.__slots__:
+        if slot not in ("__weakref__", "_version_counter"):
+            assert getattr(view, slot) == getattr(made, slot), slot
+    assert view._version_counter.value == 0 and view._version_counter is not made._version_counter
