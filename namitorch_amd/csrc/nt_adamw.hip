@@ -302,9 +302,10 @@ __device__ __forceinline__ void lean_slice_f16(const DevTensor &d, const nt_adam
 
 // BLOCK lanes per workgroup, UNROLL 4-element groups in flight per lane;
 // each workgroup takes one slice of a task (task_slice).  A whole one-wave
-// slice in the common case runs lean_slice; everything else (tensor tails,
-// unaligned tensors, deferred addends, maximize, coupled decay, lr == 0,
-// fp16 rounding, the whole-task shape) the general loop below.
+// slice in the common case runs lean_slice, one of float16 parameters
+// lean_slice_f16 when its whole launch may (MtArgs::half_lean); everything
+// else (tensor tails, unaligned tensors, deferred addends, maximize, coupled
+// decay, lr == 0, the whole-task shape) the general loop below.
 template <class P, class G, class S, class C, class R, bool HAS_COPY, int BLOCK, int UNROLL>
 __global__ __launch_bounds__(BLOCK) void adamw_mt_kernel(const DevTensor *__restrict__ tensors,
                                                          const Task *__restrict__ tasks, MtArgs args) {
@@ -521,24 +522,28 @@ constexpr size_t pass_lds_cap() {
 // +0.1 %) and 3-7 % on flat 4-64 M-element tensors, while the 16-bit layouts
 // measured up to 5 % slower with any grouping, so they keep the launch order.
 //
-// Float16 launches whose slices can all run lean_slice_f16 (half_lean_slots,
-// every tensor aligned, no deferred addend) take its kPassSliceF16 slices under an occupancy
-// cap of kPassLdsF16 bytes (16 workgroups per CU); the general loop, which
-// that cap slows by a quarter, keeps kPassSlice slices and none.
+// Float16 launches whose slices can all run lean_slice_f16 (half_lean_slots:
+// AdamW without maximize; every tensor aligned; no deferred addend) take its
+// kPassSliceF16 slices under an occupancy cap of kPassLdsF16 bytes (16
+// workgroups per CU).  The others run the general loop throughout, bound by
+// arithmetic at some 5 TB/s: Adam's coupled decay, maximize, and every tensor
+// of a list with one that is not 16-byte aligned.  The cap would slow that
+// loop by a quarter, so it keeps kPassSlice slices and none.
 template <class P, class G, class S, class C, class R, bool HAS_COPY>
 static int32_t launch_mt(nt_plan *plan, const MtArgs &args, hipStream_t stream) {
     MtArgs a = args;
     constexpr bool half = std::is_same<R, RoundF16>::value;
-    if constexpr (half) a.half_lean = plan->aligned && plan->n_incoming == 0 && half_lean_slots(args.slots, plan->max_slot + 1u) ? 1 : 0;
+    if constexpr (half)
+        a.half_lean = plan->aligned && plan->n_incoming == 0 && half_lean_slots(args.slots, plan->max_slot + 1u);
     a.split_shift = split_shift(plan, a.half_lean ? kPassSliceF16 : kPassSlice, 64);
     constexpr bool all_fp32 = std::is_same<P, TF32>::value && std::is_same<G, TF32>::value &&
                               std::is_same<S, TF32>::value && !HAS_COPY;
     a.xcd_group = all_fp32 && a.split_shift > 0 ? kFp32XcdGroup : 0u;
     if (a.split_shift > 0) {
         static_assert(kPassSlice == 64 * kVec, "one 4-element group per lane of one wave");
+        const size_t lds = a.half_lean ? kPassLdsF16 : pass_lds_cap<P, G, S>();
         adamw_mt_kernel<P, G, S, C, R, HAS_COPY, 64, 1><<<dim3((unsigned)(plan->ntasks << a.split_shift)), dim3(64),
-                                                          a.half_lean ? kPassLdsF16 : pass_lds_cap<P, G, S>(), stream>>>(plan->d_tensors,
-                                                                                             plan->d_tasks, a);
+                                                          lds, stream>>>(plan->d_tensors, plan->d_tasks, a);
     } else {
         adamw_mt_kernel<P, G, S, C, R, HAS_COPY, kBlock, kPass2Unroll><<<dim3((unsigned)plan->ntasks), dim3(kBlock), 0,
                                                                          stream>>>(plan->d_tensors, plan->d_tasks, a);

@@ -886,9 +886,9 @@ __global__ __launch_bounds__(BLOCK) void grad_apply_kernel(const DevTensor *__re
 // One gradient by its address, without a plan: what a program that reads its
 // gradients one by one after a clip queues per read (the launch is what costs
 // there: 148 bfloat16 gradients of GPT-2 clipped and read took 3.4 ms a pass
-// through one-tensor plans, 1.7 ms in this form).  A workgroup takes one iteration of the lanes:
-// 1024 float32 or 2048 16-bit elements, so that small gradients spread over
-// the chip; past the largest launch (17 G float32 or 34 G 16-bit elements) it
+// through one-tensor plans, 1.7 ms in this form).  A workgroup takes one
+// iteration of the lanes: 1024 float32 or 2048 16-bit elements, so that small
+// gradients spread over the chip; past the largest launch (17 G float32 or 34 G 16-bit elements) it
 // strides over the array.
 template <class G>
 constexpr uint64_t flat_apply_tile() { return (uint64_t)kBlock * kVec * ApplyShape<G>::unroll; }

@@ -12,7 +12,9 @@ prescaled form with a second pass whenever max|g| lies outside
 ulps rather than bit for bit: NumPy sums the prescaled squares pairwise and
 takes ``power(total, 0.5)``, whose last bit depends on the host (SVML's pow
 on AVX-512 CPUs, libm's elsewhere), so no device formula can match it on
-every host.  Other p use the prescaled form with a second pass.  The
+every host.  p = 1 and 3 of float32/float16/bfloat16 gradients take one pass
+in ``get_grad_norm``: their powers stay within float64 as well.  Every other
+p, and 1 and 3 elsewhere, use the prescaled form with a second pass.  The
 reduction order is fixed, so the result is deterministic.
 
 Clipping multiplies each gradient by ``max_norm / (norm + 1e-6)`` in
@@ -21,10 +23,10 @@ rewrite is recorded on the gradients (see ``GradTransform``) and fused into
 the next kernel that reads them.  When nothing is pending on the gradients
 and ``error_if_nonfinite`` is False, the norm, the ``coefficient < 1``
 decision and the coefficient stay on the device (``_clip_on_device``): the
-call queues two kernels and returns without waiting, and the AdamW pass
+call queues its kernels and returns without waiting, and the AdamW pass
 that follows reads the decision from the device.  ``get_grad_norm`` takes
-the same device path (``_norm_on_device``) and records nothing on the
-gradients; ``.item()`` on either result waits for it.
+the same device path (``_norm_on_device``), for every p, and records nothing
+on the gradients; ``.item()`` on either result waits for it.
 """
 
 from __future__ import annotations
