@@ -1,9 +1,8 @@
 """Host unit tests of the library's plain C++ parts — the plan-table builder,
 the caching memory pools, the GradScaler / clip decisions the finalize
 kernels make, the kernels' workgroup -> element arithmetic and the float16
-pass's — compiled
-with g++ under AddressSanitizer and UndefinedBehaviorSanitizer (no GPU
-involved)."""
+pass's divisions and roots — compiled with g++ under AddressSanitizer and
+UndefinedBehaviorSanitizer (no GPU involved)."""
 
 from __future__ import annotations
 
